@@ -394,9 +394,9 @@ def flux_div(prims, rhs, flux, increment=True):
 
 
 def flux_div_kernel(prims, flux):
-    """'fast' (LDS face-once kernel), 'specialized' (per-cell kernel compiled for
-    a composition of cent_keep<2>, pressure_diss_lr and visc_lr) or 'generic'
-    (per-cell kernel for every functor) for this array and flux."""
+    """'fast' (LDS face-once kernel on 16x16 cross-sections), 'specialized'
+    (tiled face-once kernel for every composition with compile-time code) or
+    'generic' (per-cell kernel for every functor) for this array and flux."""
     d = flux_descriptor(flux)
     kind = C.c_int()
     check(load().spd_flux_div_kernel(prims._h, C.byref(d), C.byref(kind)))

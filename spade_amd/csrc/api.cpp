@@ -169,6 +169,8 @@ int spd_ctx_create(int device, spd_ctx_t* out)
         c->c.device = device;
         SPD_HIP(hipSetDevice(device));
         init_device_scratch(device);
+        SPD_HIP(hipDeviceGetAttribute(&c->c.cus, hipDeviceAttributeMultiprocessorCount, device));
+        if (c->c.cus < 1) c->c.cus = 1;
         SPD_HIP(hipStreamCreateWithFlags(&c->c.stream, hipStreamNonBlocking));
         SPD_HIP(hipEventCreate(&c->c.ev0));
         SPD_HIP(hipEventCreate(&c->c.ev1));

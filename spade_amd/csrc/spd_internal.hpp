@@ -48,6 +48,7 @@ struct DevGeom
 struct Ctx
 {
     int device = 0;
+    int cus = 1;                  // compute units of the device
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // two pinned host buffers for the binary checkpoint, double-buffered
@@ -115,6 +116,10 @@ __host__ __device__ inline int fixup_start(const int* start, int lb)
 // ---- kernels' host launchers ----
 void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
                              bool increment, hipStream_t s);
+// the tiled kernel for the compositions of flux_div_spec_code on blocks of any
+// size and any coordinates; false (nothing launched) for others
+bool launch_flux_div_tile(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
+                          hipStream_t s);
 void launch_flux_div_fixup(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
                            hipStream_t s);
 bool launch_flux_div_fast(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
