@@ -290,14 +290,11 @@ int spd_grid_create(spd_ctx_t ctx, const spd_grid_desc* d, spd_grid_t* out)
                 if (nbr[27*D + e] >= 0) push[27*nbr[27*D + e] + e] = D;
         SPD_HIP(hipMalloc((void**)&g.d_nbr, sizeof(int)*27*dg.nblk));
         SPD_HIP(hipMalloc((void**)&g.d_push, sizeof(int)*27*dg.nblk));
-        SPD_HIP(hipMalloc((void**)&g.d_start, sizeof(int)*kFixupParts*dg.nblk));
         SPD_HIP(hipMemcpy(g.d_tables, g.h_dx.data(), sizeof(double)*3*dg.nblk, hipMemcpyHostToDevice));
         SPD_HIP(hipMemcpy(g.d_tables + 3*dg.nblk, g.h_inv_dx.data(), sizeof(double)*3*dg.nblk, hipMemcpyHostToDevice));
         SPD_HIP(hipMemcpy(g.d_tables + 6*dg.nblk, g.h_bmin.data(), sizeof(double)*3*dg.nblk, hipMemcpyHostToDevice));
         SPD_HIP(hipMemcpy(g.d_nbr, nbr.data(), sizeof(int)*27*dg.nblk, hipMemcpyHostToDevice));
         SPD_HIP(hipMemcpy(g.d_push, push.data(), sizeof(int)*27*dg.nblk, hipMemcpyHostToDevice));
-        const std::vector<int> complete((size_t)kFixupParts*dg.nblk, dg.nc[2]);
-        SPD_HIP(hipMemcpy(g.d_start, complete.data(), sizeof(int)*kFixupParts*dg.nblk, hipMemcpyHostToDevice));
         dg.dx = g.d_tables;
         dg.inv_dx = g.d_tables + 3*dg.nblk;
         dg.bmin = g.d_tables + 6*dg.nblk;
@@ -314,7 +311,6 @@ int spd_grid_destroy(spd_grid_t grid)
         SPD_HIP(hipFree(grid->g.d_tables));
         SPD_HIP(hipFree(grid->g.d_nbr));
         SPD_HIP(hipFree(grid->g.d_push));
-        SPD_HIP(hipFree(grid->g.d_start));
         if (grid->g.d_stage) SPD_HIP(hipFree(grid->g.d_stage));
         if (grid->g.d_red) SPD_HIP(hipFree(grid->g.d_red));
         if (grid->g.h_red) SPD_HIP(hipHostFree(grid->g.h_red));

@@ -1,9 +1,8 @@
 // Per-cell evaluation of every flux functor: the cells, normals and gradients
-// of a face gathered from the array, the term functions in the reference's
-// expression order, and the residual of one cell by six face evaluations
-// (pde-algs/flux-div/flux_div_basic.h:47-72).  Used by the per-cell kernels
-// and the fix-ups (flux_generic.hip) and by the tiled kernel's redo of planes
-// whose face temperatures leave the power-law series (flux_tile.hpp).
+// of a face gathered from the array, and the term functions in the reference's
+// expression order (pde-algs/flux-div/flux_div_basic.h:47-72), for the generic
+// kernel (flux_generic.hip).  The face-once kernels evaluate the same
+// expressions on their LDS windows.
 #pragma once
 #include "spd_internal.hpp"
 #include "pow_series.hpp"
@@ -17,9 +16,8 @@ struct Prim { double p, T, u, v, w; };
 __device__ inline double vel(const Prim& q, int d) { return d == 0 ? q.u : (d == 1 ? q.v : q.w); }
 
 // The power law's series and the exponent it belongs to.  Every kernel
-// evaluates x^n of a face the same way: by the series where x is in its range,
-// by the library pow elsewhere, so a face has the same bits whichever kernel
-// (LDS-staged, tiled, per-cell, fix-up) evaluates it.
+// evaluates x^n of a face the same way (pow_faces in flux_face.hpp): by the
+// series where x is in its range, by the library pow elsewhere.
 struct PowAt
 {
     double power;
@@ -595,95 +593,10 @@ __device__ __forceinline__ void f_visc(const Cell& C, const FaceIdx& f, const sp
     out[4] = -(n[0]*tau[2][0] + n[1]*tau[2][1] + n[2]*tau[2][2]);
 }
 
-// The per-cell code specialised for one composition of up to three terms
-// (cent_keep<2> / <4>, totani_lr, pressure_diss_lr, weno_t, fweno_t,
-// first_order_t, weno_fds_t, visc_lr), on any geometry.  The terms are known
-// at compile time, so with everything inlined the small arrays the term
-// functions fill (stencils, gradients, metrics) stay in registers instead of
-// the per-lane stack that the run-time dispatch of k_flux_div_generic needs.
-// The arithmetic is the same code in the same order as generic_cell, so the
-// two give the same bits.
-constexpr int TERM_KEEP4 = 19;  // cent_keep<4>; SPD_TERM_KEEP stands for cent_keep<2> here
-
-// convective terms of the tiled kernel
+// term codes beside SPD_TERM_* in flux_div_spec_code, and the convective
+// terms of the tiled kernel
+constexpr int TERM_KEEP4 = 19;  // cent_keep<4>; SPD_TERM_KEEP stands for cent_keep<2> there
 enum { CV_NONE = 0, CV_KEEP2, CV_KEEP4, CV_TOTANI, CV_WENO, CV_FWENO, CV_FIRST, CV_FDS };
-
-template <int K>
-__device__ inline void eval_static(const Cell& C, const FaceIdx& f, const spd_flux_term& t, double R, double gam,
-                                   double out[5])
-{
-    if constexpr (K == SPD_TERM_KEEP) f_keep(C, f, 2, R, gam, out);
-    else if constexpr (K == TERM_KEEP4) f_keep(C, f, 4, R, gam, out);
-    else if constexpr (K == SPD_TERM_TOTANI) f_totani(C, f, R, gam, out);
-    else if constexpr (K == SPD_TERM_PDISS) f_pdiss(C, f, t, R, gam, out);
-    else if constexpr (K == SPD_TERM_WENO) f_weno(C, f, t, R, gam, out);
-    else if constexpr (K == SPD_TERM_FWENO) f_fweno(C, f, t, R, gam, out);
-    else if constexpr (K == SPD_TERM_FIRST) f_first(C, f, R, gam, out);
-    else if constexpr (K == SPD_TERM_WENO_FDS) f_weno_fds(C, f, t, R, gam, out);
-    else f_visc(C, f, t, R, gam, out);
-}
-
-template <int K>
-__device__ inline void add_static(const Cell& C, const FaceIdx& f, const spd_flux_term& t, double R, double gam,
-                                  double acc[5])
-{
-    asm volatile("" ::: "memory");       // nor of one term for the next
-    double z[5];
-    eval_static<K>(C, f, t, R, gam, z);
-    for (int n = 0; n < 5; ++n) { z[n] += acc[n]; acc[n] = z[n]; }
-}
-
-// F0 + (F1 + F2): the last term first, then each earlier one plus the sum
-template <int T0, int T1, int T2>
-__device__ inline void spec_face(const Cell& C, const FaceIdx& f, const spd_flux_desc& F, double acc[5])
-{
-    if constexpr (T2 != 0)
-    {
-        eval_static<T2>(C, f, F.terms[2], F.R, F.gamma, acc);
-        add_static<T1>(C, f, F.terms[1], F.R, F.gamma, acc);
-        add_static<T0>(C, f, F.terms[0], F.R, F.gamma, acc);
-    }
-    else if constexpr (T1 != 0)
-    {
-        eval_static<T1>(C, f, F.terms[1], F.R, F.gamma, acc);
-        add_static<T0>(C, f, F.terms[0], F.R, F.gamma, acc);
-    }
-    else eval_static<T0>(C, f, F.terms[0], F.R, F.gamma, acc);
-}
-
-template <int T0, int T1, int T2>
-__device__ inline void spec_cell(const DevGeom& G, const double* __restrict__ prims, double* __restrict__ rhs,
-                                 const spd_flux_desc& F, const PowAt& ps, int increment, int i, int j, int k, int lb)
-{
-    Cell C{&G, prims + (long long)lb*G.sb, lb, &ps};
-    double jac = 1.0;
-    if (!G.identity)
-    {
-        double xi[3]; cell_xi(G, lb, i, j, k, xi);
-        jac = 1.0/(map_deriv(G, 0, xi[0])*map_deriv(G, 1, xi[1])*map_deriv(G, 2, xi[2]));
-    }
-    double relem[5];
-    for (int v = 0; v < 5; ++v) relem[v] = increment ? rhs[cell_index(G, lb, v, i, j, k)] : 0.0;
-    #pragma clang loop unroll(disable)
-    for (int idir = 0; idir < 3; ++idir)
-    {
-        const double inv_dx = 1.0/G.dx[3*lb + idir];
-        #pragma clang loop unroll(disable)
-        for (int pm = 0; pm < 2; ++pm)
-        {
-            // nothing of a face is kept for the next one: six faces' geometry and
-            // stencils at once would not fit the registers
-            asm volatile("" ::: "memory");
-            FaceIdx f{idir, i, j, k};
-            if (pm == 1) { if (idir == 0) f.i++; else if (idir == 1) f.j++; else f.k++; }
-            double acc[5];
-            spec_face<T0, T1, T2>(C, f, F, acc);
-            const double s = jac*(1.0 - 2.0*pm)*inv_dx;
-            for (int n = 0; n < 5; ++n) { acc[n] *= s; relem[n] += acc[n]; }
-        }
-    }
-    for (int v = 0; v < 5; ++v) rhs[cell_index(G, lb, v, i, j, k)] = relem[v];
-}
 
 // The series of a composition's first power-law viscosity (an exponent no
 // other term matches when there is none)

@@ -75,13 +75,57 @@ __device__ inline double div_const(double a, double b, double y)
     return __builtin_fma(r, y, q0);
 }
 
-// x^n of the power law by the branch-free binomial series; `bad` records a
-// lane whose x is outside the series range (its block is then completed by
-// the fix-up kernel with the library pow, from that plane on)
-__device__ inline double pow_law(const FastCfg& C, double x, bool& bad)
+// (T/T_ref)^n of the power law for N faces of a thread, from the sums of the
+// temperatures at their sides: by the branch-free binomial series, and where a
+// lane's x is outside its range by the library pow -- one cold loop behind a
+// wave-uniform branch, placed where little else is live, so that the hot path
+// keeps its registers and no later launch has to complete a block.  (A launch
+// for that after every flux_div and stage cost 4-8 us and a gap even with
+// nothing to do: 64^3 ten steps 754 -> 670 us without it, channel ten steps
+// 5.81 -> 5.10 ms, channel flux_div 128.5 -> 117.5 us, with the shallower
+// prefetch of the 16 x 16 kernel that makes room for it.)  Every kernel evaluates a face's x^n this way, so a face has
+// the same bits whichever kernel evaluates it.
+// Faces from M on are evaluated where `more` (the same in a whole wave) says so.
+template <int M, int N>
+__device__ inline void pow_faces(const PowSeries& ps, const double (&x)[N], double n, bool more, double (&pw)[N])
 {
-    bad |= !C.ps.in_range(x);
-    return C.ps.eval(x);
+    bool bad = false;
+    #pragma unroll
+    for (int e = 0; e < M; ++e)
+    {
+        bad |= !ps.in_range(x[e]);
+        pw[e] = ps.eval(x[e]);
+    }
+    if (M < N && more)
+    {
+        #pragma unroll
+        for (int e = M; e < N; ++e)
+        {
+            bad |= !ps.in_range(x[e]);
+            pw[e] = ps.eval(x[e]);
+        }
+    }
+    if (__builtin_expect(__any(bad), 0))
+    {
+        #pragma clang loop unroll(disable)
+        for (int f = 0; f < N; ++f)
+        {
+            double xf = x[0];
+            #pragma unroll
+            for (int e = 1; e < N; ++e) xf = f == e ? x[e] : xf;
+            if (ps.in_range(xf)) continue;
+            const double r = pow(xf, n);
+            #pragma unroll
+            for (int e = 0; e < N; ++e) pw[e] = f == e ? r : pw[e];
+        }
+    }
+}
+
+// x = T/T_ref of a face
+__device__ inline double pow_arg(const FastCfg& C, double ST)
+{
+    const double Tf = ST*0.5;
+    return C.t_ref_one ? Tf : div_const(Tf, C.T_ref, C.inv_T_ref);
 }
 
 // ducros_t::get_sensor (state_sensor.h:32-42); g[c][q], q = u, v, w
@@ -183,17 +227,16 @@ __device__ inline double wale_s(const Cfg& C, double pf, double Tf, const double
 }
 
 // visc_lr row D for the unit normal of identity coordinates (viscous.h:39-112),
-// times the composition scale s (carried by mu, beta and the conductivity).
+// times the composition scale s (carried by mu, beta and the conductivity);
+// pw: the face's (T/T_ref)^n (pow_faces) with the power law.
 template <int D, class S, bool MAP, class Cfg>
 __device__ inline void visc_s(const Cfg& C, const FaceSums& f, const double g[3][3], double gT, double nf,
-                              double F[5], bool& bad)
+                              double F[5], double pw)
 {
     double mu, visc2, cond;
     if constexpr (S::law == SPD_LAW_POWER)
     {
-        const double Tf = f.ST*0.5;
-        const double x = C.t_ref_one ? Tf : div_const(Tf, C.T_ref, C.inv_T_ref);
-        mu    = C.mu_ref_s*pow_law(C, x, bad);
+        mu    = C.mu_ref_s*pw;
         visc2 = -0.66666666667*mu;
         cond  = C.spec_heat*div_const(mu, C.prandtl, C.inv_prandtl);
     }
@@ -260,11 +303,11 @@ __device__ inline void visc_s(const Cfg& C, const FaceSums& f, const double g[3]
 // jac (1 - 2 pm)/dx (flux_div_basic.h:66-68).
 template <int D, class S, bool MAP, class Cfg>
 __device__ inline void face_product(const Cfg& C, const CellV& L, const CellV& R, const double g[3][3], double gT,
-                                    double idx, const double mt[3], double P[5], bool& bad)
+                                    double idx, const double mt[3], double P[5], double pw)
 {
     const FaceSums f = face_sums(L, R);
     double s8[5];
-    if (S::vs) visc_s<D, S, MAP>(C, f, g, gT, mt[2], s8, bad);
+    if (S::vs) visc_s<D, S, MAP>(C, f, g, gT, mt[2], s8, pw);
     if (S::pd)
     {
         double z[5];

@@ -13,9 +13,8 @@
 // 18x18 plane with one halo layer (ring of three slots), and for planes k and
 // k+1 the p, T, rho, e needed as left/right states of the faces.
 //
-// Power law: x^n comes from a binomial series valid near x = 1.  A block
-// with a face temperature outside its range stops at that plane, and
-// k_flux_fixup (flux_generic.hip) completes it with the library pow.
+// Power law: x^n comes from a binomial series valid near x = 1, and from the
+// library pow for faces outside its range (pow_faces).
 //
 // Arithmetic follows the reference's expression order exactly
 // (navier-stokes/convective.h:117-184, 212-245; viscous.h:39-112;
@@ -125,8 +124,7 @@ struct StageArgs
 // one are isothermal walls whose ghosts are formed from the mirrored cells)
 template <int KEEP, int PDISS, int VISC, bool INC, bool MAP, int STG = 0>
 __global__ void __launch_bounds__(256, 2)
-k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, FastCfg C,
-            int* __restrict__ start, StageArgs A, int split)
+k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, FastCfg C, StageArgs A, int split)
 {
     using S = Spec<KEEP, PDISS, VISC>;
     static_assert(!(STG && INC), "a fused stage writes a fresh residual");
@@ -134,7 +132,6 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     // face, staged for whole-row writes (flushed after the next barrier)
     __shared__ double sXs[STG ? sizeof(XStage)/sizeof(double) : 1];
     XStage& xs = *reinterpret_cast<XStage*>(sXs);
-    __shared__ int sBad[2];               // a face of plane k is outside the pow series range (by parity)
     // mapped coordinates: d x_a / d xi_a of this block at cell centres -1 .. 16
     // and at faces 0 .. 16 of each axis, from the same map_deriv as the
     // per-cell kernels (so the same bits)
@@ -152,19 +149,13 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
 
     // zsplit 2 or 4: that many workgroups per block, each marching over its
     // share of the planes [k0, k1) with its own window prologue (fewer, shorter tail rounds when
-    // the block count is not a multiple of the resident workgroups); each
-    // records the first plane it left to the fix-up in its own d_start entry.
-    // The fix-up redoes the block from the first of them to the end, which
-    // overwrites whatever the other half wrote there: the same planes the
-    // one-workgroup launch leaves, so the same bits (overwrite mode only)
+    // the block count is not a multiple of the resident workgroups)
     // split: workgroups per block in the low byte, bit 8 set for XCD runs
     const int zsplit = split & 0xff;
     const int w = (split & 0x100) ? xcd_run_order(blockIdx.x, G.nblk*zsplit) : blockIdx.x;
     const int lb = w/zsplit, half = w - lb*zsplit;
     const int k0 = half*(G.nc[2]/zsplit), k1 = k0 + G.nc[2]/zsplit;
-    int* __restrict__ my_start = start + kFixupParts*lb + half;
     const int tid = threadIdx.x;
-    if (half == 0 && tid < kFixupParts && tid >= zsplit) start[kFixupParts*lb + tid] = G.nc[2];
     const int i = tid & 15, j = tid >> 4;
     const double ix = G.inv_dx[3*lb + 0], iy = G.inv_dx[3*lb + 1], iz = G.inv_dx[3*lb + 2];
     const bool yonly = MAP && G.map_kind[0] == SPD_MAP_IDENTITY && G.map_kind[2] == SPD_MAP_IDENTITY;
@@ -205,6 +196,10 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     else if (tid < 64) { hi = tid - 48; hj = 16; }
     else if (tid < 68) { const int c = tid - 64; hi = (c & 1) ? 16 : -1; hj = (c & 2) ? 16 : -1; }
     const int pown = lpos(i, j), phalo = lpos(hi, hj);
+    // left and right cell of the block-boundary face of a lane of wave 2 (x,
+    // row tid - 128) or 3 (y, column tid - 192); the other lanes' own cell
+    const int pbl = (tid >= 128 && tid < 144) ? lpos(15, tid - 128) : (tid >= 192 && tid < 208) ? lpos(tid - 192, 15) : pown;
+    const int pbr = (tid >= 128 && tid < 144) ? lpos(16, tid - 128) : (tid >= 192 && tid < 208) ? lpos(tid - 192, 16) : pown;
 
     // column bases at plane k = 0; plane k is base + k*stride (the own column
     // and the residual are core columns, a halo column with hi = -1 or 16 is
@@ -277,34 +272,31 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     #pragma unroll
     for (int n = 0; n < 5; ++n) rin[n] = INC ? Rown[k0*plane + n*sv] : 0.0;
 
-    // prologue: planes k0-1, k0, k0+1 resident; planes k0+2 and k0+3 in flight
-    // (two raw register sets used alternately, so a plane's load is never
-    // copied and waiting for it never waits for the later one)
+    // prologue: planes k0-1, k0, k0+1 resident; plane k0+2 in flight (one
+    // plane ahead is a whole plane's arithmetic, 4 us, ahead of its use; a
+    // second one only took 20 registers the fused stages spilled for)
     const CellV prev = cell(load_own(k0 - 1));
     const CellV cur0 = cell(load_own(k0));
     const CellV nxt0 = cell(load_own(k0 + 1));
-    Raw nA{}, nB{}, hA{}, hB{};
-    if (k0 + 2 <= k1) nA = load_own(k0 + 2);
-    if (k0 + 3 <= k1) nB = load_own(k0 + 3);
+    Raw nr{}, hr{};
+    if (k0 + 2 <= k1) nr = load_own(k0 + 2);
     put_vel(ring[0], pown, prev);
     put_vel(ring[1], pown, cur0); put_sca(sS[0], pown, cur0);
     put_vel(ring[2], pown, nxt0); put_sca(sS[1], pown, nxt0);
-    if (tid == 0) { sBad[0] = 0; sBad[1] = 0; }
     if (has_halo)
     {
         put_vel(ring[0], phalo, cell(load_halo(k0 - 1)));
         const CellV h0 = cell(load_halo(k0)), h1 = cell(load_halo(k0 + 1));
         put_vel(ring[1], phalo, h0); put_sca(sS[0], phalo, h0);
         put_vel(ring[2], phalo, h1); put_sca(sS[1], phalo, h1);
-        if (k0 + 2 <= k1) hA = load_halo(k0 + 2);
-        if (k0 + 3 <= k1) hB = load_halo(k0 + 3);
+        if (k0 + 2 <= k1) hr = load_halo(k0 + 2);
     }
     lds_barrier();
 
     // mapped coordinates: this column's d x / d xi along x and y (cell centres)
     const double m0i = MAP ? sMc[0][i + 1] : 1.0, m1j = MAP ? sMc[1][j + 1] : 1.0;
     double zlo[5];
-    bool bad = false;                     // carried into plane 0's check
+    constexpr bool power = S::vs && S::law == SPD_LAW_POWER;
     {
         double g[3][3], gT, mt[3] = {1.0, 1.0, 1.0};
         grads_z<S>(ring[0], ring[1], pown, prev, cur0, ix, iy, iz, g, gT);
@@ -321,13 +313,18 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             }
             grads_map<2>(G, g, gT, mf, m0i, m1j);
         }
-        face_product<2, S, MAP>(C, prev, cur0, g, gT, iz, mt, zlo, bad);
+        double pw[1] = {1.0};
+        if constexpr (power)
+        {
+            const double x[1] = {pow_arg(C, prev.T + cur0.T)};
+            pow_faces<1>(C.ps, x, C.power, false, pw);
+        }
+        face_product<2, S, MAP>(C, prev, cur0, g, gT, iz, mt, zlo, pw[0]);
     }
 
     // One plane k: every face, the residual of its cells, and the entry of
-    // plane k+2 (from nr / hr, which are then refilled with plane k+4).
-    // Returns false when the block must be left to the fix-up kernel.
-    auto plane_step = [&](int k, Raw& nr, Raw& hr) -> bool
+    // plane k+2 (from nr / hr, which are then refilled with plane k+3).
+    auto plane_step = [&](int k)
     {
         // the x pushes staged by plane k-1 (visible since its last barrier;
         // the staging buffer is refilled only after this plane's first barrier)
@@ -339,6 +336,18 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
         // the cells of this column in planes k and k+1, from the window
         const CellV cur = cell_from_lds(sk, s0, pown);
         const CellV nxt = cell_from_lds(sS[(k + 1) & 1], sp, pown);
+        // the power law of the thread's three faces and, in waves 2 and 3, of
+        // its block-boundary face
+        double pw[4] = {1.0, 1.0, 1.0, 1.0};
+        if constexpr (power)
+        {
+            const double* sT = sk + HP;
+            double x[4] = {pow_arg(C, sT[pown - 1] + cur.T), pow_arg(C, sT[pown - HX] + cur.T),
+                           pow_arg(C, cur.T + nxt.T), 1.0};
+            const bool closing = __builtin_amdgcn_readfirstlane(tid) >= 128;
+            if (closing) x[3] = pow_arg(C, sT[pbl] + sT[pbr]);
+            pow_faces<3>(C.ps, x, C.power, closing, pw);
+        }
         double zhi[5];
         // this cell's own low x- and y-face products (the LDS copies serve
         // the neighbour cells that share those faces); the residual reads
@@ -370,7 +379,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 }
                 grads_map<0>(G, g, gT, mf, m1j, m2k);
             }
-            face_product<0, S, MAP>(C, L, cur, g, gT, ix, mt, px, bad);
+            face_product<0, S, MAP>(C, L, cur, g, gT, ix, mt, px, pw[0]);
             for (int n = 0; n < 5; ++n) sFx[n][j*17 + i] = px[n];
         }
         {
@@ -391,7 +400,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 }
                 grads_map<1>(G, g, gT, mf, m2k, m0i);
             }
-            face_product<1, S, MAP>(C, L, cur, g, gT, iy, mt, py, bad);
+            face_product<1, S, MAP>(C, L, cur, g, gT, iy, mt, py, pw[1]);
             for (int n = 0; n < 5; ++n) sFy[n][j*16 + i] = py[n];
         }
         {
@@ -410,7 +419,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 }
                 grads_map<2>(G, g, gT, mf, m0i, m1j);
             }
-            face_product<2, S, MAP>(C, cur, nxt, g, gT, iz, mt, zhi, bad);
+            face_product<2, S, MAP>(C, cur, nxt, g, gT, iz, mt, zhi, pw[2]);
         }
         if (tid >= 128 && tid < 144)
         {
@@ -432,7 +441,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 }
                 grads_map<0>(G, g, gT, mf, m1, m2k);
             }
-            face_product<0, S, MAP>(C, L, Rr, g, gT, ix, mt, P, bad);
+            face_product<0, S, MAP>(C, L, Rr, g, gT, ix, mt, P, pw[3]);
             for (int n = 0; n < 5; ++n) sFx[n][jj*17 + 16] = P[n];
         }
         if (tid >= 192 && tid < 208)
@@ -455,7 +464,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 }
                 grads_map<1>(G, g, gT, mf, m2k, m0);
             }
-            face_product<1, S, MAP>(C, L, Rr, g, gT, iy, mt, P, bad);
+            face_product<1, S, MAP>(C, L, Rr, g, gT, iy, mt, P, pw[3]);
             for (int n = 0; n < 5; ++n) sFy[n][16*16 + ii] = P[n];
         }
         #pragma unroll
@@ -474,17 +483,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 for (int v = 0; v < 5; ++v) rprev[t][v] = A.r[t][co + v*sv];
             }
         }
-        if (bad) sBad[k & 1] = 1;
         lds_barrier();
-        if (sBad[k & 1])
-        {
-            // some face of plane k needs the library pow: planes k .. nz-1 are
-            // left to the fix-up kernel (nothing of them was written)
-            if (tid == 0) *my_start = k;
-            return false;
-        }
-        if (tid == 0) sBad[(k + 1) & 1] = 0;
-        bad = false;
 
         // rhs of cell (i,j,k): faces in the order x-, x+, y-, y+, z-, z+
         // (flux_div_basic.h:54-72; the high faces enter as -P)
@@ -565,7 +564,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
         if (k + 1 < k1)
         {
             // plane k+2 (<= k1) enters into the ring slot of plane k-1 and the
-            // parity buffer of plane k; its raw registers take plane k+4
+            // parity buffer of plane k; its raw registers take plane k+3
             double* s_new = ring[0];
             ring[0] = ring[1]; ring[1] = ring[2]; ring[2] = s_new;
             double* t_new = sS[k & 1];
@@ -576,25 +575,19 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             }
             const CellV c2 = cell(nr);
             put_vel(s_new, pown, c2); put_sca(t_new, pown, c2);
-            if (k + 4 <= k1) nr = load_own(k + 4);
+            if (k + 3 <= k1) nr = load_own(k + 3);
             if (has_halo)
             {
                 const CellV h = cell(hr);
                 put_vel(s_new, phalo, h); put_sca(t_new, phalo, h);
-                if (k + 4 <= k1) hr = load_halo(k + 4);
+                if (k + 3 <= k1) hr = load_halo(k + 3);
             }
         }
         lds_barrier();
-        return true;
     };
 
-    for (int k = k0; k < k1; k += 2)
-    {
-        if (!plane_step(k, nA, hA)) return;
-        if (k + 1 < k1 && !plane_step(k + 1, nB, hB)) return;
-    }
+    for (int k = k0; k < k1; ++k) plane_step(k);
     if (STG && A.push_ghosts) flush_x(G, A.push, A.qout, xs, lb, k1 - 1);   // after the last plane's closing barrier
-    if (tid == 0) *my_start = nz;
 }
 
 // Workgroups per block (1, 2 or 4), each marching over an equal share of the
@@ -611,14 +604,10 @@ int fast_zsplit(const Grid& g)
         const int zs = e[0] == '4' ? 4 : (e[0] == '2' ? 2 : 1);
         return ok(zs) ? zs : 1;
     }
-    static int cus[64] = {};
-    const int dev = g.ctx->device;
-    if (dev < 0 || dev >= 64) return 1;
-    if (!cus[dev]) SPD_HIP(hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev));
-    const long slots = 2L*(cus[dev] > 0 ? cus[dev] : 1), nb = g.geom.nblk;
+    const long slots = 2L*g.ctx->cus, nb = g.geom.nblk;
     int best = 1;
     double best_cost = 1e300;
-    for (int zs = 1; zs <= kFixupParts; zs *= 2)
+    for (int zs = 1; zs <= 4; zs *= 2)
     {
         if (!ok(zs)) continue;
         const double rounds = (double)((zs*nb + slots - 1)/slots);
@@ -647,24 +636,21 @@ int fast_xcd_runs(bool shared_reads)
 template <int KEEP, int PDISS, int VISC>
 void launch_fast(const Grid& g, const double* prims, double* rhs, const FastCfg& C, bool increment, hipStream_t s)
 {
-    // increment mode keeps one workgroup per block: the fix-up redoes a block
-    // from its first flagged plane on, which would add the other half's
-    // already-written planes twice
-    const int zs = increment ? 1 : fast_zsplit(g);
+    const int zs = fast_zsplit(g);
     const int xr = fast_xcd_runs(zs > 1) ? 0x100 : 0;
     const bool map = !g.geom.identity;
     if (increment && map)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, true, true>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, g.d_start, StageArgs{}, zs | xr);
+                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
     else if (increment)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, true, false>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, g.d_start, StageArgs{}, zs | xr);
+                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
     else if (map)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, g.d_start, StageArgs{}, zs | xr);
+                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
     else
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, g.d_start, StageArgs{}, zs | xr);
+                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
     SPD_LAUNCH_CHECK();
 }
 
@@ -688,16 +674,16 @@ void launch_fast_stage(const Grid& g, const double* qin, double* rhs, const Fast
     const int xr = fast_xcd_runs(read_neighbours || zs > 1) ? 0x100 : 0;
     if (!g.geom.identity && read_neighbours)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true, 2>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, g.d_start, A, zs | xr);
+                           g.geom, qin, rhs, C, A, zs | xr);
     else if (!g.geom.identity)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true, 1>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, g.d_start, A, zs | xr);
+                           g.geom, qin, rhs, C, A, zs | xr);
     else if (read_neighbours)
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false, 2>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, g.d_start, A, zs | xr);
+                           g.geom, qin, rhs, C, A, zs | xr);
     else
         hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false, 1>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, g.d_start, A, zs | xr);
+                           g.geom, qin, rhs, C, A, zs | xr);
     SPD_LAUNCH_CHECK();
 }
 
@@ -779,9 +765,6 @@ bool launch_flux_div_fast(const Grid& g, const double* prims, double* rhs, const
         case 4: ok = dispatch_visc<1, 1>(vs, g, prims, rhs, C, increment, s); break;
         case 5: ok = dispatch_visc<1, 2>(vs, g, prims, rhs, C, increment, s); break;
     }
-    // power law: blocks with a face temperature outside the pow series range
-    // are completed by the per-cell kernel (an early exit per block when none)
-    if (ok && vs == 1 + SPD_LAW_POWER) launch_flux_div_fixup(g, prims, rhs, f, increment, s);
     return ok;
 }
 
@@ -847,33 +830,7 @@ bool launch_flux_stage_fast(const Grid& g, const double* qin, double* qout, doub
         case 4: ok = dispatch_visc_stage<1, 1>(vs, g, qin, rhs, C, A, read_neighbours, s); break;
         case 5: ok = dispatch_visc_stage<1, 2>(vs, g, qin, rhs, C, A, read_neighbours, s); break;
     }
-    if (!ok) return false;
-    // power law: blocks with a face temperature outside the pow series range
-    // were left from that plane on; their residual (into rhs) and stage
-    // (qin -> qout) are completed here (early exits per block when none)
-    if (vs == 1 + SPD_LAW_POWER)
-    {
-        // the per-cell fix-up reads its block's ghost cells: after a
-        // neighbour-read stage they may be stale, so the flagged blocks pull
-        // theirs first (what an exchange copies; the others exit at once)
-        // (and, on the walled channel, fill their wall ghost slabs from the
-        // cells just pulled).  One launch does all of it for the compositions
-        // with a specialised per-cell kernel (every one the fast kernel
-        // takes); SPD_SPLIT_FIXUP=1 keeps the three launches
-        const double* r[3] = {rprev && nr > 1 ? rprev[0] : nullptr, rprev && nr > 2 ? rprev[1] : nullptr, nullptr};
-        r[nr - 1] = rhs;
-        bool merged = false;
-        if (const char* e = getenv("SPD_SPLIT_FIXUP"); !(e && e[0] == '1'))
-            merged = launch_stage_fixup_spec(g, const_cast<double*>(qin), qout, rhs, f, r, coef, nr, gamma, R,
-                                             read_neighbours, A.wall_y, t_wall, s);
-        if (!merged)
-        {
-            if (read_neighbours) launch_exchange_flagged(g, const_cast<double*>(qin), s, A.wall_y, t_wall);
-            launch_flux_div_fixup(g, qin, rhs, f, false, s);
-            launch_stage_fixup(g, qin, qout, r, coef, nr, gamma, R, s);
-        }
-    }
-    return true;
+    return ok;
 }
 
 } // namespace spd

@@ -62,15 +62,6 @@ struct TileSpec : Spec<(CONV == CV_KEEP2), PDISS, VISC>
     static constexpr int SS = (2 + extra) | 1;                   // doubles per scalar record
     static constexpr bool power = Base::vs && Base::law == SPD_LAW_POWER;
     static constexpr double scale = CONV == CV_KEEP2 ? 8.0 : 1.0;
-    // term codes of flux_cell.hpp's spec_cell
-    static constexpr int tc = CONV == CV_KEEP2 ? int(SPD_TERM_KEEP) : CONV == CV_KEEP4 ? TERM_KEEP4
-        : CONV == CV_TOTANI ? int(SPD_TERM_TOTANI) : CONV == CV_WENO ? int(SPD_TERM_WENO)
-        : CONV == CV_FWENO ? int(SPD_TERM_FWENO) : CONV == CV_FIRST ? int(SPD_TERM_FIRST)
-        : CONV == CV_FDS ? int(SPD_TERM_WENO_FDS) : 0;
-    static constexpr int tp = PDISS ? int(SPD_TERM_PDISS) : 0, tv = VISC ? int(SPD_TERM_VISC) : 0;
-    static constexpr int T0 = tc ? tc : (tp ? tp : tv);
-    static constexpr int T1 = tc ? (tp ? tp : tv) : (tp ? tv : 0);
-    static constexpr int T2 = tc && tp ? tv : 0;
 };
 
 // x: KEEP / Totani {rho, e}; WENO, first order {rho/2, E, E + p/rho, sigma rho}
@@ -172,20 +163,20 @@ constexpr double kKeep4A = (2.0/6.0)*(2.0/1.0)*1/1.0, kKeep4B = (2.0/24.0)*(2.0/
 // Composed flux F (times S::scale) through a face of direction D.  q[0..n-1]:
 // the cells at offsets -1, 0 (narrow) or -2 .. 1 (wide); nc: their normal
 // factors, nf: the face's (all 1 on identity coordinates); g, gT: the face
-// gradient where the composition has one.
+// gradient and pw the power law's (T/T_ref)^n where the composition has them.
 template <int D, class S>
 __device__ inline void visc_face(const TileCfg& C, const TCell& A, const TCell& B, double nf, const double g[3][3],
-                                 double gT, double z[5], bool& bad)
+                                 double gT, double z[5], double pw)
 {
     FaceSums f;
     f.SU = A.u + B.u; f.SV = A.v + B.v; f.SW = A.w + B.w;
     f.SP = A.p + B.p; f.ST = A.T + B.T; f.K = 0.0;
-    visc_s<D, S, true>(C, f, g, gT, nf, z, bad);
+    visc_s<D, S, true>(C, f, g, gT, nf, z, pw);
 }
 
 template <int D, class S>
 __device__ inline void face_flux(const TileCfg& C, const TCell* q, const double* nc, double nf, const double g[3][3],
-                                 double gT, double F[5], bool& bad)
+                                 double gT, double F[5], double pw)
 {
     constexpr int l = S::wide ? 1 : 0, r = l + 1;
     const TCell& A = q[l];
@@ -195,7 +186,7 @@ __device__ inline void face_flux(const TileCfg& C, const TCell* q, const double*
     double z[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if constexpr (S::vs && S::conv != CV_KEEP2 && S::conv != CV_NONE)
     {
-        visc_face<D, S>(C, A, B, nf, g, gT, z, bad);
+        visc_face<D, S>(C, A, B, nf, g, gT, z, pw);
         if constexpr (S::wide)
         {
             #pragma unroll
@@ -207,7 +198,7 @@ __device__ inline void face_flux(const TileCfg& C, const TCell* q, const double*
     {
         const CellV L{A.p, A.T, A.u, A.v, A.w, A.x[0], A.x[1]}, R{B.p, B.T, B.u, B.v, B.w, B.x[0], B.x[1]};
         const double mt[3] = {nc[l], nc[r], nf};
-        face_product<D, S, true>(C, L, R, g, gT, 1.0, mt, F, bad);
+        face_product<D, S, true>(C, L, R, g, gT, 1.0, mt, F, pw);
         return;
     }
     else if constexpr (S::conv == CV_TOTANI)
@@ -426,11 +417,9 @@ struct TileLds
 
 template <class S, bool MAP>
 __global__ void __launch_bounds__(256, 2) __attribute__((flatten))
-k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, TileCfg C,
-                     spd_flux_desc F, PowAt ps, int increment)
+k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, TileCfg C, int increment)
 {
     extern __shared__ double lds[];
-    __shared__ int sBad[2];                   // a face of plane k left the pow series (by parity)
     constexpr int H = S::H, SS = S::SS, NQ = S::wide ? 4 : 2, l = S::wide ? 1 : 0;
     constexpr double sc = 1.0/S::scale;
     constexpr int Y = 2*H + 1;                // (z tables start at plane k0 - H)
@@ -569,12 +558,9 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         put_vel(rm, pos, q_m); put_vel(rz, pos, q_0); put_vel(rp, pos, q_1);
         put_sca(pos, c0);
     }
-    if (tid == 0) { sBad[0] = 0; sBad[1] = 0; }
     lds_barrier();
 
     const double m0i = MAP ? tX[i + H] : 1.0, m1j = MAP ? tY[j + H] : 1.0;
-    bool bad = false;
-    unsigned long long redo = 0;              // planes (from k0) left to the redo below
     double zlo[5];
     // z-face between planes kf-1 and kf: normals of its cells and of the face
     auto z_normals = [&](int kf, double nc[NQ], double& nf, double& mf)
@@ -597,8 +583,13 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             nf = nrm_at(mf, jac_at(m0i, m1j, mf));
         }
     };
-    if (active)
     {
+        double pw[1] = {1.0};
+        if constexpr (S::power)
+        {
+            const double x[1] = {pow_arg(C, cm.T + c0.T)};
+            pow_faces<1>(C.ps, x, C.power, false, pw);
+        }
         double g[3][3] = {}, gT = 0.0, nc[NQ], nf = 1.0, mf = 1.0;
         #pragma unroll
         for (int m = 0; m < NQ; ++m) nc[m] = 1.0;
@@ -611,12 +602,12 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         if constexpr (S::wide)
         {
             const TCell q[4] = {derive<S>(C, below), cm, c0, c1};
-            face_flux<2, S>(C, q, nc, nf, g, gT, zlo, bad);
+            face_flux<2, S>(C, q, nc, nf, g, gT, zlo, pw[0]);
         }
         else
         {
             const TCell q[2] = {cm, c0};
-            face_flux<2, S>(C, q, nc, nf, g, gT, zlo, bad);
+            face_flux<2, S>(C, q, nc, nf, g, gT, zlo, pw[0]);
         }
         #pragma unroll
         for (int n = 0; n < 5; ++n) { if (!MAP) zlo[n] = zlo[n]*(sc*iz); }
@@ -628,16 +619,43 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     const int by = tid - (nw - 1)*64;
     const int bx = wi*wj <= (nw - 1)*64 ? by : tid - max(nw - 2, 0)*64;
 
+    const bool closing = __builtin_amdgcn_readfirstlane(tid) >= 64*max(nw - 2, 0);   // a wave with closing faces
+
     for (int k = k0; k < k1; ++k)
     {
         const Win W{rm, rz, rp, py};
         const double m2k = MAP ? tZ[k - k0 + H] : 1.0;
         const double jc = MAP ? (yonly ? tY[nY + j + H] : jac_at(m0i, m1j, m2k)) : 1.0;
+        // the power law of the thread's three faces and of a closing face
+        double pw[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
+        if constexpr (S::power)
+        {
+            const double* t = sS + 1;
+            double x[5] = {1.0, 1.0, 1.0, 1.0, 1.0};
+            if (active)
+            {
+                const double T0 = t[SS*pos];
+                x[0] = pow_arg(C, t[SS*(pos - 1)] + T0);
+                x[1] = pow_arg(C, t[SS*(pos - PX)] + T0);
+                x[2] = pow_arg(C, T0 + c1.T);
+            }
+            if (bx >= 0 && bx < wj)
+            {
+                const int p = (bx + H)*PX + (wi + H);
+                x[3] = pow_arg(C, t[SS*(p - 1)] + t[SS*p]);
+            }
+            if (by >= 0 && by < wi)
+            {
+                const int p = (wj + H)*PX + (by + H);
+                x[4] = pow_arg(C, t[SS*(p - PX)] + t[SS*p]);
+            }
+            pow_faces<3>(C.ps, x, C.power, closing, pw);
+        }
         double px[5], pyf[5], zhi[5], rin[5];
         const long long ro = blk + own + (long long)k*plane;
         TCell c2{};
         // x-face below cell ci (tile index) of row jj
-        auto x_face = [&](int ci, int jj, int p, const TCell* mine, double P[5])
+        auto x_face = [&](int ci, int jj, int p, const TCell* mine, double pf, double P[5])
         {
             TCell q[NQ];
             #pragma unroll
@@ -668,12 +686,12 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
                 }
                 if constexpr (S::grad) grads_map<0>(G, g, gT, mf, m1, m2k);
             }
-            face_flux<0, S>(C, q, nc, nf, g, gT, P, bad);
+            face_flux<0, S>(C, q, nc, nf, g, gT, P, pf);
             #pragma unroll
             for (int n = 0; n < 5; ++n) { if (!MAP) P[n] = P[n]*(sc*ix); }
         };
         // y-face below cell (ii, cj)
-        auto y_face = [&](int ii, int cj, int p, const TCell* mine, double P[5])
+        auto y_face = [&](int ii, int cj, int p, const TCell* mine, double pf, double P[5])
         {
             TCell q[NQ];
             #pragma unroll
@@ -704,7 +722,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
                 }
                 if constexpr (S::grad) grads_map<1>(G, g, gT, mf, m2k, m0);
             }
-            face_flux<1, S>(C, q, nc, nf, g, gT, P, bad);
+            face_flux<1, S>(C, q, nc, nf, g, gT, P, pf);
             #pragma unroll
             for (int n = 0; n < 5; ++n) { if (!MAP) P[n] = P[n]*(sc*iy); }
         };
@@ -714,11 +732,11 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         // used, and the z-face, with its plane k+2, comes last
         if (active)
         {
-            x_face(i, j, pos, S::wide ? nullptr : &c0, px);
+            x_face(i, j, pos, S::wide ? nullptr : &c0, pw[0], px);
             #pragma unroll
             for (int n = 0; n < 5; ++n) sFx[(j*(C.wi + 1) + i)*5 + n] = px[n];
             if constexpr (S::wide) __builtin_amdgcn_sched_barrier(0);
-            y_face(i, j, pos, S::wide ? nullptr : &c0, pyf);
+            y_face(i, j, pos, S::wide ? nullptr : &c0, pw[1], pyf);
             #pragma unroll
             for (int n = 0; n < 5; ++n) sFy[(j*C.wi + i)*5 + n] = pyf[n];
             if constexpr (S::wide) __builtin_amdgcn_sched_barrier(0);
@@ -726,14 +744,14 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         if (bx >= 0 && bx < wj)
         {
             double P[5];
-            x_face(wi, bx, (bx + H)*PX + (wi + H), nullptr, P);
+            x_face(wi, bx, (bx + H)*PX + (wi + H), nullptr, pw[3], P);
             #pragma unroll
             for (int n = 0; n < 5; ++n) sFx[(bx*(C.wi + 1) + wi)*5 + n] = P[n];
         }
         if (by >= 0 && by < wi)
         {
             double P[5];
-            y_face(by, wj, (wj + H)*PX + (by + H), nullptr, P);
+            y_face(by, wj, (wj + H)*PX + (by + H), nullptr, pw[4], P);
             #pragma unroll
             for (int n = 0; n < 5; ++n) sFy[(wj*C.wi + by)*5 + n] = P[n];
         }
@@ -757,12 +775,12 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             if constexpr (S::wide)
             {
                 const TCell q[4] = {cm, c0, c1, c2};
-                face_flux<2, S>(C, q, nc, nf, g, gT, zhi, bad);
+                face_flux<2, S>(C, q, nc, nf, g, gT, zhi, pw[2]);
             }
             else
             {
                 const TCell q[2] = {c0, c1};
-                face_flux<2, S>(C, q, nc, nf, g, gT, zhi, bad);
+                face_flux<2, S>(C, q, nc, nf, g, gT, zhi, pw[2]);
             }
             #pragma unroll
             for (int n = 0; n < 5; ++n) { if (!MAP) zhi[n] = zhi[n]*(sc*iz); keep_here(zhi[n]); }
@@ -771,13 +789,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         // the other waves covers its latency
         #pragma unroll
         for (int n = 0; n < 5; ++n) rin[n] = increment && active ? rhs[ro + n*sv] : 0.0;
-        if (S::power && bad) sBad[k & 1] = 1;
         lds_barrier();
-        // the next plane shares this one's high z-face
-        if (S::power && sBad[k & 1]) redo |= 3ull << (k - k0);
-        const bool left = S::power && ((redo >> (k - k0)) & 1);
-        if (S::power && tid == 0) sBad[(k + 1) & 1] = 0;
-        bad = false;
         if (active)
         {
             // faces in the order x-, x+, y-, y+, z-, z+ (flux_div_basic.h:54-72)
@@ -801,7 +813,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
                     r += yl;     r -= yh;
                     r += zlo[n]; r -= zhi[n];
                 }
-                if (!left) rhs[ro + n*sv] = r;
+                rhs[ro + n*sv] = r;
                 zlo[n] = zhi[n];
             }
         }
@@ -836,26 +848,6 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             }
         }
         lds_barrier();
-    }
-
-    if constexpr (S::power)
-    {
-        // planes with a face temperature outside the pow series: nothing of
-        // them was written, and the per-cell code (library pow where the series
-        // does not reach) does them now
-        if (!redo) return;
-        __shared__ DevGeom sG;                // run-time indexed by the per-cell code
-        __shared__ spd_flux_desc sF;
-        __shared__ PowAt sP;
-        if (tid == 0) { sG = G; sF = F; sP = ps; }
-        __syncthreads();
-        for (int k = k0; k < k1; ++k)
-        {
-            if (!((redo >> (k - k0)) & 1) || !active) continue;
-            int ri = i0 + i, rj = j0 + j, rb = lb;   // opaque: nothing of a cell is hoisted out of the plane loop
-            asm volatile("" : "+v"(ri), "+v"(rj), "+v"(rb));
-            spec_cell<S::T0, S::T1, S::T2>(sG, prims, rhs, sF, sP, increment, ri, rj, k, rb);
-        }
     }
 }
 
@@ -940,12 +932,11 @@ void launch_tile(const Grid& g, const double* prims, double* rhs, const spd_flux
     TileCfg C = tile_cfg(f, S::scale);
     C.wi = p.wi; C.wj = p.wj; C.tx = p.tx; C.ty = p.ty; C.zs = p.zs;
     const dim3 grid((unsigned)(p.tx*p.ty*p.zs*G.nblk)), block((unsigned)p.nt);
-    const PowAt ps = pow_of(f);
     const int inc = increment ? 1 : 0;
     if (map)
-        hipLaunchKernelGGL((k_flux_div_spec_tile<S, true>), grid, block, p.lds, s, G, prims, rhs, C, f, ps, inc);
+        hipLaunchKernelGGL((k_flux_div_spec_tile<S, true>), grid, block, p.lds, s, G, prims, rhs, C, inc);
     else
-        hipLaunchKernelGGL((k_flux_div_spec_tile<S, false>), grid, block, p.lds, s, G, prims, rhs, C, f, ps, inc);
+        hipLaunchKernelGGL((k_flux_div_spec_tile<S, false>), grid, block, p.lds, s, G, prims, rhs, C, inc);
     SPD_LAUNCH_CHECK();
 }
 

@@ -33,33 +33,6 @@ k_exchange(DevGeom G, const int* __restrict__ nbr, double* __restrict__ a, int x
     exchange_item(G, nbr, a, lb, part*blockDim.x + threadIdx.x);
 }
 
-// The exchange of the blocks the LDS-staged flux kernel left to the fix-up
-// (only[lb] < nz): one workgroup per block, the others exit at once.  With
-// wall_y (isothermal walls on both y faces), a flagged block at a wall then
-// fills that wall's ghost slab, as the wall fill after an exchange would: the
-// slab mirrors rows of the block, x- and z-ghost cells included, which this
-// workgroup has just written (visible to it after the barrier)
-__global__ void __launch_bounds__(256)
-k_exchange_flagged(DevGeom G, const int* __restrict__ nbr, double* __restrict__ a, const int* __restrict__ only,
-                   int wall_y, double t_wall)
-{
-    const int lb = blockIdx.x;
-    if (fixup_start(only, lb) >= G.nc[2]) return;
-    const int items = exchange_items(G);
-    for (int t = threadIdx.x; t < items; t += blockDim.x) exchange_item(G, nbr, a, lb, t);
-    if (!wall_y) return;
-    const int by = (lb / G.nb[0]) % G.nb[1];
-    const bool low = by == 0, high = by == G.nb[1] - 1;
-    if (!low && !high) return;                       // the same for the whole workgroup
-    __syncthreads();
-    const int n = G.N[0]*G.ng*G.N[2];
-    for (int pm = 0; pm < 2; ++pm)
-    {
-        if (pm == 0 ? !low : !high) continue;
-        for (int c = threadIdx.x; c < n; c += blockDim.x) wall_cell(G, a, lb, 1, pm, c, t_wall);
-    }
-}
-
 __global__ void __launch_bounds__(256)
 k_wall_fill(DevGeom G, double* __restrict__ a, int idir, int pm, double t_wall)
 {
@@ -318,13 +291,6 @@ void launch_exchange(const Grid& g, double* a, hipStream_t s)
     int xr = 1;
     if (const char* e = getenv("SPD_EXCH_XCD")) xr = e[0] == '1' ? 1 : 0;
     hipLaunchKernelGGL(k_exchange, dim3((items + 255)/256, g.geom.nblk), dim3(256), 0, s, g.geom, g.d_nbr, a, xr);
-    SPD_LAUNCH_CHECK();
-}
-
-void launch_exchange_flagged(const Grid& g, double* a, hipStream_t s, int wall_y, double t_wall)
-{
-    hipLaunchKernelGGL(k_exchange_flagged, dim3(g.geom.nblk), dim3(256), 0, s, g.geom, g.d_nbr, a,
-                       (const int*)g.d_start, wall_y, t_wall);
     SPD_LAUNCH_CHECK();
 }
 

@@ -105,43 +105,6 @@ k_rk_opt_s2(DevGeom G, double* __restrict__ q, const double* __restrict__ r0, co
     push_result(G, push, q, ci, qq, xs);
 }
 
-// The stage of the cells a fused flux + stage launch left to the fix-up: the
-// planes k >= start[lb] of each block, whose residual (C.r[C.n - 1]) the
-// per-cell fix-up kernel has just written.  Reads qin, writes qout and its
-// pushed ghosts, with k_rk_transform's arithmetic.  One 256-thread workgroup
-// per 16 x 16 block cross-section, planes in order; blocks with nothing to
-// redo exit at once.
-__global__ void __launch_bounds__(256)
-k_stage_fixup(DevGeom G, const double* __restrict__ qin, double* __restrict__ qout, Coefs C, double gamma,
-              double R, const int* __restrict__ push, const int* __restrict__ start)
-{
-    __shared__ XStage xs;
-    const int lb = blockIdx.x;
-    for (int k = fixup_start(start, lb); k < G.nc[2]; ++k)
-    {
-        const CellIt ci{(int)(threadIdx.x & 15), (int)(threadIdx.x >> 4), k, lb};
-        double qq[5], cons[5];
-        long long idx[5];
-        for (int v = 0; v < 5; ++v) { idx[v] = core_index(G, lb, v, ci.i, ci.j, k); qq[v] = qin[idx[v]]; }
-        p2c(gamma, R, qq, cons);
-        #pragma unroll
-        for (int s = 0; s < kMaxStages; ++s)
-        {
-            if (s >= C.n || C.c[s] == 0.0) continue;
-            double inc[5];
-            for (int v = 0; v < 5; ++v) inc[v] = C.c[s]*C.r[s][idx[v]];
-            for (int v = 0; v < 5; ++v) cons[v] += inc[v];
-        }
-        c2p(gamma, R, cons, qq);
-        for (int v = 0; v < 5; ++v) qout[idx[v]] = qq[v];
-        push_ghosts(G, push, qout, ci, qq, true);
-        stage_x(G, xs, ci, qq);
-        lds_barrier();
-        flush_x(G, push, qout, xs, lb, k);
-        lds_barrier();
-    }
-}
-
 // grid_array::operator*=(scalar) (grid/grid_array.h:369-379): every stored double
 __global__ void __launch_bounds__(256)
 k_array_scale(double* __restrict__ a, long long n, double s)
@@ -200,18 +163,6 @@ void launch_rk_transform_stage(const Grid& g, double* q, const double* const* r,
     for (int j = 0; j < nr; ++j) { C.r[j] = r[j]; C.c[j] = coef[j]; }
     hipLaunchKernelGGL(k_rk_transform, interior_blocks(g.geom), dim3(256), 0, s, g.geom, q, C, gamma, R,
                        push ? g.d_push : nullptr);
-    SPD_LAUNCH_CHECK();
-}
-
-void launch_stage_fixup(const Grid& g, const double* qin, double* qout, const double* const* r, const double* coef,
-                        int nr, double gamma, double R, hipStream_t s)
-{
-    if (nr < 1 || nr > kMaxStages) throw ArgError{"a stage combines 1.." + std::to_string(kMaxStages) + " residuals"};
-    Coefs C{};
-    C.n = nr;
-    for (int j = 0; j < nr; ++j) { C.r[j] = r[j]; C.c[j] = coef[j]; }
-    hipLaunchKernelGGL(k_stage_fixup, dim3((unsigned)g.geom.nblk), dim3(256), 0, s, g.geom, qin, qout, C, gamma, R,
-                       g.d_push, g.d_start);
     SPD_LAUNCH_CHECK();
 }
 

@@ -66,7 +66,6 @@ struct Grid
     double* d_tables = nullptr;   // dx, inv_dx, bmin
     int* d_nbr = nullptr;         // [27*lb + e] source block for ghost region e, -1 = not exchanged
     int* d_push = nullptr;        // [27*lb + e] block whose ghost region e block lb feeds, -1 = none
-    int* d_start = nullptr;       // [lb] first plane the LDS-staged flux kernel left to the fix-up kernel
     double* d_stage = nullptr;    // host-layout staging for upload / download (stage_blocks blocks), lazily allocated
     int stage_blocks = 0;
     double* d_red = nullptr;      // reduction partials, 2 nblk + 1 doubles, lazily allocated
@@ -101,18 +100,6 @@ __device__ inline void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The first plane of block lb left to the fix-up kernels by the LDS-staged
-// flux kernel (nz when none): that kernel may split a block's planes between
-// up to kFixupParts workgroups, each recording the first plane it left in its
-// own entry (d_start holds kFixupParts ints per block)
-constexpr int kFixupParts = 4;
-__host__ __device__ inline int fixup_start(const int* start, int lb)
-{
-    int m = start[kFixupParts*lb];
-    for (int e = 1; e < kFixupParts; ++e) m = start[kFixupParts*lb + e] < m ? start[kFixupParts*lb + e] : m;
-    return m;
-}
-
 // ---- kernels' host launchers ----
 void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
                              bool increment, hipStream_t s);
@@ -120,15 +107,12 @@ void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, co
 // size and any coordinates; false (nothing launched) for others
 bool launch_flux_div_tile(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
                           hipStream_t s);
-void launch_flux_div_fixup(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
-                           hipStream_t s);
 bool launch_flux_div_fast(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
                           bool increment, hipStream_t s);
 bool flux_div_fast_eligible(const Grid& g, const spd_flux_desc& f);
 // One transform-aware RK stage fused with flux_div on the fast kernel:
 // qout <- c2p(p2c(qin) + sum_{j < nr-1} coef[j] r[j] + coef[nr-1] L(qin)) on
-// interior cells; L(qin) is also written to rhs when store_rhs (and, for the
-// planes left to the fix-up, always).  push: the ghosts the result feeds are
+// interior cells; L(qin) is also written to rhs when store_rhs.  push: the ghosts the result feeds are
 // written into qout (else qout's ghost cells are left alone).
 // read_neighbours: L(qin) takes its halo from the neighbour blocks' interiors
 // instead of qin's ghost cells (x and z periodic, y periodic or isothermal
@@ -149,17 +133,6 @@ int flux_div_spec_code(const spd_flux_desc& f);
 // the composition contains a hybrid_scheme_t term
 bool flux_has_hybrid(const spd_flux_desc& f);
 void launch_exchange(const Grid& g, double* a, hipStream_t s);
-// The fix-up of a fused stage in one launch for the compositions with a
-// specialised per-cell kernel: per block with d_start[lb] < nz, (pull) its
-// ghosts and (wall_y) wall slabs, the residual of its planes from there into
-// rhs, and their stage qin -> qout with r[0..nr-1], r[nr-1] = rhs; false
-// (nothing launched) for the other compositions
-bool launch_stage_fixup_spec(const Grid& g, double* qin, double* qout, double* rhs, const spd_flux_desc& f,
-                             const double* const* r, const double* coef, int nr, double gamma, double R,
-                             bool pull, int wall_y, double t_wall, hipStream_t s);
-// the exchange of the blocks with d_start[lb] < nz only (the others exit at
-// once); wall_y: those at a y wall then fill its isothermal ghost slab at t_wall
-void launch_exchange_flagged(const Grid& g, double* a, hipStream_t s, int wall_y = 0, double t_wall = 0.0);
 void launch_wall_fill(const Grid& g, double* a, int face, double t_wall, hipStream_t s);
 // boundary_fill over the faces of face_mask (bit 2*dir+pm), one launch per face in face order
 void launch_fill_extrap(const Grid& g, double* a, int face_mask, int order, hipStream_t s);
@@ -173,11 +146,6 @@ void launch_soa_to_aos(const Grid& g, const double* a, double* stage, int lb0, i
 // push = false leaves every ghost cell alone (interior update only)
 void launch_rk_transform_stage(const Grid& g, double* q, const double* const* r, const double* coef, int nr,
                                double gamma, double R, hipStream_t s, bool push = true);
-// the same stage, qin -> qout (ghosts pushed into qout), for the planes
-// k >= d_start[lb] of each block only (the cells a fused launch left to the
-// fix-up); 16 x 16 block cross-sections
-void launch_stage_fixup(const Grid& g, const double* qin, double* qout, const double* const* r, const double* coef,
-                        int nr, double gamma, double R, hipStream_t s);
 // grid_array element-wise operations: scale every stored double; a (+|-)= b on
 // interior cells; convert_state in place (every stored cell or the interior)
 void launch_array_scale(const Grid& g, double* a, double sc, hipStream_t s);

@@ -1,8 +1,8 @@
 // Per-cell pieces of a transform-aware RK stage shared by the stage kernels
-// (rk.hip), the fused flux + stage kernel (flux_fast.hip) and its fix-up
-// (flux_generic.hip): the prim<->cons transforms, the fused exchange that
-// writes a stage result into the ghost cells of the neighbour blocks, the
-// exchange of one block's ghost cells and the isothermal wall mirror.  Compiled without contraction, so
+// (rk.hip) and the fused flux + stage kernel (flux_fast.hip): the prim<->cons
+// transforms and the fused exchange that writes a stage result into the ghost
+// cells of the neighbour blocks; and the exchange of one block's ghost cells
+// and the isothermal wall mirror (grid_ops.hip).  Compiled without contraction, so
 // both kernels round every expression alike.
 #pragma once
 #include "spd_internal.hpp"
