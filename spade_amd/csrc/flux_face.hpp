@@ -372,6 +372,17 @@ __device__ inline void grads_map(const DevGeom& G, double g[3][3], double& gT, d
     if (G.map_kind[B] != SPD_MAP_IDENTITY) for (int b = 0; b < 3; ++b) g[B][b] = g[B][b]/mB;
 }
 
+// The same when only y is mapped: m = d y / d eta at the face point and
+// rm = RN(1/m), tabulated per block, so that each quotient costs three
+// operations instead of a division (div_const: the same bits)
+template <int D>
+__device__ inline void grads_map_y(double g[3][3], double& gT, double m, double rm)
+{
+    #pragma unroll
+    for (int b = 0; b < 3; ++b) g[1][b] = div_const(g[1][b], m, rm);
+    if (D == 1) gT = div_const(gT, m, rm);
+}
+
 // metric() of a diagonal map at a point with derivatives m0, m1, m2: jac =
 // 1/(m0 m1 m2), normal component D = 1/(m_D jac) (core/coord_system.h:250-302)
 __device__ inline double jac_at(double m0, double m1, double m2) { return 1.0/(m0*m1*m2); }

@@ -122,7 +122,8 @@ struct StageArgs
 // 2 fused stage, halo from the neighbour blocks' interiors (every ghost
 // region has a source block, or, in the mapped kernel, the y regions without
 // one are isothermal walls whose ghosts are formed from the mirrored cells)
-template <int KEEP, int PDISS, int VISC, bool INC, bool MAP, int STG = 0>
+// MAP: 0 identity coordinates, 1 only y mapped, 2 any diagonal map
+template <int KEEP, int PDISS, int VISC, bool INC, int MAP, int STG = 0>
 __global__ void __launch_bounds__(256, 2)
 k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, FastCfg C, StageArgs A, int split)
 {
@@ -140,8 +141,9 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     // every face normal and Jacobian depends on the row alone, tabulated per
     // block with the same expressions: sY[0][r] = jac at cell row r - 1,
     // sY[1][r] = its normal factor 1/(1 jac), sY[2][r] = the y-face normal
-    // factor of a cell row, sY[3][f] = the y-face normal factor at face f
-    __shared__ double sY[MAP ? 4 : 1][18];
+    // factor of a cell row, sY[3][f] = the y-face normal factor at face f,
+    // sY[4][r] and sY[5][f] = 1/(d y / d eta) there
+    __shared__ double sY[MAP == 1 ? 6 : 1][18];
     __shared__ double sU[3][3*HP];        // u, v, w of planes k-1, k, k+1 (ring)
     __shared__ double sS[2][4*HP];        // p, T, rho, e of planes k, k+1 (by parity)
     __shared__ double sFx[5][16*17];      // x-face products, faces i = 0..16 of row j
@@ -158,7 +160,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     const int tid = threadIdx.x;
     const int i = tid & 15, j = tid >> 4;
     const double ix = G.inv_dx[3*lb + 0], iy = G.inv_dx[3*lb + 1], iz = G.inv_dx[3*lb + 2];
-    const bool yonly = MAP && G.map_kind[0] == SPD_MAP_IDENTITY && G.map_kind[2] == SPD_MAP_IDENTITY;
+    constexpr bool yonly = MAP == 1;
     if constexpr (MAP)
     {
         if (tid < 54)
@@ -166,10 +168,11 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             const int a = tid/18, c = tid % 18 - 1;
             const double m = map_deriv(G, a, G.bmin[3*lb + a] + (c + 0.5)*G.dx[3*lb + a]);
             sMc[a][c + 1] = m;
-            if (a == 1)
+            if (yonly && a == 1)
             {
                 const double jc = jac_at(1.0, m, 1.0);
                 sY[0][c + 1] = jc; sY[1][c + 1] = nrm_at(1.0, jc); sY[2][c + 1] = nrm_at(m, jc);
+                sY[4][c + 1] = 1.0/m;
             }
         }
         else if (tid < 105)
@@ -177,7 +180,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             const int a = (tid - 54)/17, c = (tid - 54) % 17;
             const double m = map_deriv(G, a, G.bmin[3*lb + a] + ((c + 0.5) - 0.5)*G.dx[3*lb + a]);
             sMf[a][c] = m;
-            if (a == 1) sY[3][c] = nrm_at(m, jac_at(1.0, m, 1.0));
+            if (yonly && a == 1) { sY[3][c] = nrm_at(m, jac_at(1.0, m, 1.0)); sY[5][c] = 1.0/m; }
         }
     }
     const int nz = G.nc[2];
@@ -304,14 +307,15 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
         {
             // face k0 - 1/2: L = plane k0 - 1, R = plane k0
             const double mL = sMc[2][k0], mR = sMc[2][k0 + 1], mf = sMf[2][k0];
-            if (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
+            if constexpr (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
             else
             {
                 mt[0] = nrm_at(mL, jac_at(m0i, m1j, mL));
                 mt[1] = nrm_at(mR, jac_at(m0i, m1j, mR));
                 mt[2] = nrm_at(mf, jac_at(m0i, m1j, mf));
             }
-            grads_map<2>(G, g, gT, mf, m0i, m1j);
+            if constexpr (yonly) grads_map_y<2>(g, gT, m1j, sY[4][j + 1]);
+            else grads_map<2>(G, g, gT, mf, m0i, m1j);
         }
         double pw[1] = {1.0};
         if constexpr (power)
@@ -319,7 +323,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             const double x[1] = {pow_arg(C, prev.T + cur0.T)};
             pow_faces<1>(C.ps, x, C.power, false, pw);
         }
-        face_product<2, S, MAP>(C, prev, cur0, g, gT, iz, mt, zlo, pw[0]);
+        face_product<2, S, (MAP != 0)>(C, prev, cur0, g, gT, iz, mt, zlo, pw[0]);
     }
 
     // One plane k: every face, the residual of its cells, and the entry of
@@ -370,16 +374,17 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             if constexpr (MAP)
             {
                 const double mL = sMc[0][i], mf = sMf[0][i];
-                if (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
+                if constexpr (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
                 else
                 {
                     mt[0] = nrm_at(mL, jac_at(mL, m1j, m2k));
                     mt[1] = nrm_at(m0i, jc);
                     mt[2] = nrm_at(mf, jac_at(mf, m1j, m2k));
                 }
-                grads_map<0>(G, g, gT, mf, m1j, m2k);
+                if constexpr (yonly) grads_map_y<0>(g, gT, m1j, sY[4][j + 1]);
+                else grads_map<0>(G, g, gT, mf, m1j, m2k);
             }
-            face_product<0, S, MAP>(C, L, cur, g, gT, ix, mt, px, pw[0]);
+            face_product<0, S, (MAP != 0)>(C, L, cur, g, gT, ix, mt, px, pw[0]);
             for (int n = 0; n < 5; ++n) sFx[n][j*17 + i] = px[n];
         }
         {
@@ -391,16 +396,17 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             if constexpr (MAP)
             {
                 const double mL = sMc[1][j], mf = sMf[1][j];
-                if (yonly) { mt[0] = sY[2][j]; mt[1] = sY[2][j + 1]; mt[2] = sY[3][j]; }
+                if constexpr (yonly) { mt[0] = sY[2][j]; mt[1] = sY[2][j + 1]; mt[2] = sY[3][j]; }
                 else
                 {
                     mt[0] = nrm_at(mL, jac_at(m0i, mL, m2k));
                     mt[1] = nrm_at(m1j, jc);
                     mt[2] = nrm_at(mf, jac_at(m0i, mf, m2k));
                 }
-                grads_map<1>(G, g, gT, mf, m2k, m0i);
+                if constexpr (yonly) grads_map_y<1>(g, gT, mf, sY[5][j]);
+                else grads_map<1>(G, g, gT, mf, m2k, m0i);
             }
-            face_product<1, S, MAP>(C, L, cur, g, gT, iy, mt, py, pw[1]);
+            face_product<1, S, (MAP != 0)>(C, L, cur, g, gT, iy, mt, py, pw[1]);
             for (int n = 0; n < 5; ++n) sFy[n][j*16 + i] = py[n];
         }
         {
@@ -410,16 +416,17 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             if constexpr (MAP)
             {
                 const double mR = sMc[2][k + 2], mf = sMf[2][k + 1];
-                if (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
+                if constexpr (yonly) { mt[0] = mt[1] = mt[2] = sY[1][j + 1]; }
                 else
                 {
                     mt[0] = nrm_at(m2k, jc);
                     mt[1] = nrm_at(mR, jac_at(m0i, m1j, mR));
                     mt[2] = nrm_at(mf, jac_at(m0i, m1j, mf));
                 }
-                grads_map<2>(G, g, gT, mf, m0i, m1j);
+                if constexpr (yonly) grads_map_y<2>(g, gT, m1j, sY[4][j + 1]);
+                else grads_map<2>(G, g, gT, mf, m0i, m1j);
             }
-            face_product<2, S, MAP>(C, cur, nxt, g, gT, iz, mt, zhi, pw[2]);
+            face_product<2, S, (MAP != 0)>(C, cur, nxt, g, gT, iz, mt, zhi, pw[2]);
         }
         if (tid >= 128 && tid < 144)
         {
@@ -432,16 +439,17 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             if constexpr (MAP)
             {
                 const double m1 = sMc[1][jj + 1], mL = sMc[0][16], mR = sMc[0][17], mf = sMf[0][16];
-                if (yonly) { mt[0] = mt[1] = mt[2] = sY[1][jj + 1]; }
+                if constexpr (yonly) { mt[0] = mt[1] = mt[2] = sY[1][jj + 1]; }
                 else
                 {
                     mt[0] = nrm_at(mL, jac_at(mL, m1, m2k));
                     mt[1] = nrm_at(mR, jac_at(mR, m1, m2k));
                     mt[2] = nrm_at(mf, jac_at(mf, m1, m2k));
                 }
-                grads_map<0>(G, g, gT, mf, m1, m2k);
+                if constexpr (yonly) grads_map_y<0>(g, gT, m1, sY[4][jj + 1]);
+                else grads_map<0>(G, g, gT, mf, m1, m2k);
             }
-            face_product<0, S, MAP>(C, L, Rr, g, gT, ix, mt, P, pw[3]);
+            face_product<0, S, (MAP != 0)>(C, L, Rr, g, gT, ix, mt, P, pw[3]);
             for (int n = 0; n < 5; ++n) sFx[n][jj*17 + 16] = P[n];
         }
         if (tid >= 192 && tid < 208)
@@ -455,16 +463,17 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             if constexpr (MAP)
             {
                 const double m0 = sMc[0][ii + 1], mL = sMc[1][16], mR = sMc[1][17], mf = sMf[1][16];
-                if (yonly) { mt[0] = sY[2][16]; mt[1] = sY[2][17]; mt[2] = sY[3][16]; }
+                if constexpr (yonly) { mt[0] = sY[2][16]; mt[1] = sY[2][17]; mt[2] = sY[3][16]; }
                 else
                 {
                     mt[0] = nrm_at(mL, jac_at(m0, mL, m2k));
                     mt[1] = nrm_at(mR, jac_at(m0, mR, m2k));
                     mt[2] = nrm_at(mf, jac_at(m0, mf, m2k));
                 }
-                grads_map<1>(G, g, gT, mf, m2k, m0);
+                if constexpr (yonly) grads_map_y<1>(g, gT, mf, sY[5][16]);
+                else grads_map<1>(G, g, gT, mf, m2k, m0);
             }
-            face_product<1, S, MAP>(C, L, Rr, g, gT, iy, mt, P, pw[3]);
+            face_product<1, S, (MAP != 0)>(C, L, Rr, g, gT, iy, mt, P, pw[3]);
             for (int n = 0; n < 5; ++n) sFy[n][16*16 + ii] = P[n];
         }
         #pragma unroll
@@ -638,19 +647,19 @@ void launch_fast(const Grid& g, const double* prims, double* rhs, const FastCfg&
 {
     const int zs = fast_zsplit(g);
     const int xr = fast_xcd_runs(zs > 1) ? 0x100 : 0;
-    const bool map = !g.geom.identity;
-    if (increment && map)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, true, true>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
-    else if (increment)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, true, false>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
-    else if (map)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
-    else
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, prims, rhs, C, StageArgs{}, zs | xr);
+    auto go = [&](auto kernel)
+    {
+        hipLaunchKernelGGL(kernel, dim3(g.geom.nblk*zs), dim3(256), 0, s, g.geom, prims, rhs, C, StageArgs{}, zs | xr);
+    };
+    switch (map_variant(g.geom) + (increment ? 3 : 0))
+    {
+        case 0: go(k_flux_fast<KEEP, PDISS, VISC, false, 0>); break;
+        case 1: go(k_flux_fast<KEEP, PDISS, VISC, false, 1>); break;
+        case 2: go(k_flux_fast<KEEP, PDISS, VISC, false, 2>); break;
+        case 3: go(k_flux_fast<KEEP, PDISS, VISC, true, 0>); break;
+        case 4: go(k_flux_fast<KEEP, PDISS, VISC, true, 1>); break;
+        case 5: go(k_flux_fast<KEEP, PDISS, VISC, true, 2>); break;
+    }
     SPD_LAUNCH_CHECK();
 }
 
@@ -672,18 +681,19 @@ void launch_fast_stage(const Grid& g, const double* qin, double* rhs, const Fast
 {
     const int zs = fast_zsplit(g);
     const int xr = fast_xcd_runs(read_neighbours || zs > 1) ? 0x100 : 0;
-    if (!g.geom.identity && read_neighbours)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true, 2>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, A, zs | xr);
-    else if (!g.geom.identity)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, true, 1>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, A, zs | xr);
-    else if (read_neighbours)
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false, 2>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, A, zs | xr);
-    else
-        hipLaunchKernelGGL((k_flux_fast<KEEP, PDISS, VISC, false, false, 1>), dim3(g.geom.nblk*zs), dim3(256), 0, s,
-                           g.geom, qin, rhs, C, A, zs | xr);
+    auto go = [&](auto kernel)
+    {
+        hipLaunchKernelGGL(kernel, dim3(g.geom.nblk*zs), dim3(256), 0, s, g.geom, qin, rhs, C, A, zs | xr);
+    };
+    switch (map_variant(g.geom) + (read_neighbours ? 3 : 0))
+    {
+        case 0: go(k_flux_fast<KEEP, PDISS, VISC, false, 0, 1>); break;
+        case 1: go(k_flux_fast<KEEP, PDISS, VISC, false, 1, 1>); break;
+        case 2: go(k_flux_fast<KEEP, PDISS, VISC, false, 2, 1>); break;
+        case 3: go(k_flux_fast<KEEP, PDISS, VISC, false, 0, 2>); break;
+        case 4: go(k_flux_fast<KEEP, PDISS, VISC, false, 1, 2>); break;
+        case 5: go(k_flux_fast<KEEP, PDISS, VISC, false, 2, 2>); break;
+    }
     SPD_LAUNCH_CHECK();
 }
 

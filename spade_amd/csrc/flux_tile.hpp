@@ -411,11 +411,12 @@ struct TileLds
         fy = fx + 5*(wi + 1)*wj;
         tab = fy + 5*wi*(wj + 1);
         total = tab;
-        if (map) total += (wi + 2*H) + 4*(wj + 2*H) + (share + 2*H + 1) + (wi + 1) + 2*(wj + 1) + (share + 1);
+        if (map) total += (wi + 2*H) + 5*(wj + 2*H) + (share + 2*H + 1) + (wi + 1) + 3*(wj + 1) + (share + 1);
     }
 };
 
-template <class S, bool MAP>
+// MAP: 0 identity coordinates, 1 only y mapped, 2 any diagonal map
+template <class S, int MAP>
 __global__ void __launch_bounds__(256, 2) __attribute__((flatten))
 k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, TileCfg C, int increment)
 {
@@ -451,13 +452,13 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     // is mapped (x and z derivatives 1.0 exactly) Jacobians and normals depend
     // on the row alone and are tabulated with the same expressions
     double* tX = lds + Z.tab;                 // centres x
-    double* tY = tX + (C.wi + 2*H);           // centres y, Jacobian, normal (x, z faces), normal (y faces)
-    double* tZ = tY + 4*(C.wj + 2*H);         // centres z, from plane k0 - H
+    double* tY = tX + (C.wi + 2*H);           // centres y, Jacobian, normal (x, z faces), normal (y faces), 1/centre
+    double* tZ = tY + 5*(C.wj + 2*H);         // centres z, from plane k0 - H
     double* fX = tZ + (share + Y);
-    double* fY = fX + (C.wi + 1);             // faces y, normal at a y-face
-    double* fZ = fY + 2*(C.wj + 1);           // faces z, from plane k0
+    double* fY = fX + (C.wi + 1);             // faces y, normal at a y-face, 1/face
+    double* fZ = fY + 3*(C.wj + 1);           // faces z, from plane k0
     const int nY = C.wj + 2*H, nYf = C.wj + 1;
-    const bool yonly = MAP && G.map_kind[0] == SPD_MAP_IDENTITY && G.map_kind[2] == SPD_MAP_IDENTITY;
+    constexpr bool yonly = MAP == 1;
     if constexpr (MAP)
     {
         for (int t = tid; t < wi + 2*H; t += blockDim.x)
@@ -468,12 +469,12 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         {
             const double m = map_deriv(G, 1, G.bmin[3*lb + 1] + ((j0 + t - H) + 0.5)*G.dx[3*lb + 1]);
             const double jc = jac_at(1.0, m, 1.0);
-            tY[t] = m; tY[nY + t] = jc; tY[2*nY + t] = nrm_at(1.0, jc); tY[3*nY + t] = nrm_at(m, jc);
+            tY[t] = m; tY[nY + t] = jc; tY[2*nY + t] = nrm_at(1.0, jc); tY[3*nY + t] = nrm_at(m, jc); tY[4*nY + t] = 1.0/m;
         }
         for (int t = tid; t <= wj; t += blockDim.x)
         {
             const double m = map_deriv(G, 1, G.bmin[3*lb + 1] + (((j0 + t) + 0.5) - 0.5)*G.dx[3*lb + 1]);
-            fY[t] = m; fY[nYf + t] = nrm_at(m, jac_at(1.0, m, 1.0));
+            fY[t] = m; fY[nYf + t] = nrm_at(m, jac_at(1.0, m, 1.0)); fY[2*nYf + t] = 1.0/m;
         }
         for (int t = tid; t < k1 - k0 + 2*H; t += blockDim.x)
             tZ[t] = map_deriv(G, 2, G.bmin[3*lb + 2] + ((k0 + t - H) + 0.5)*G.dx[3*lb + 2]);
@@ -566,7 +567,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     auto z_normals = [&](int kf, double nc[NQ], double& nf, double& mf)
     {
         mf = fZ[kf - k0];
-        if (yonly)
+        if constexpr (yonly)
         {
             #pragma unroll
             for (int m = 0; m < NQ; ++m) nc[m] = tY[2*nY + j + H];
@@ -597,7 +598,8 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
         if constexpr (S::grad)
         {
             tile_grads_z<S>(rm, rz, py, 3*pos, cm, c0, ix, iy, iz, g, gT);
-            if constexpr (MAP) grads_map<2>(G, g, gT, mf, m0i, m1j);
+            if constexpr (yonly) grads_map_y<2>(g, gT, m1j, tY[4*nY + j + H]);
+            else if constexpr (MAP) grads_map<2>(G, g, gT, mf, m0i, m1j);
         }
         if constexpr (S::wide)
         {
@@ -668,7 +670,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             if constexpr (MAP)
             {
                 const double m1 = tY[jj + H], mf = fX[ci];
-                if (yonly)
+                if constexpr (yonly)
                 {
                     #pragma unroll
                     for (int m = 0; m < NQ; ++m) nc[m] = tY[2*nY + jj + H];
@@ -684,7 +686,8 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
                     }
                     nf = nrm_at(mf, jac_at(mf, m1, m2k));
                 }
-                if constexpr (S::grad) grads_map<0>(G, g, gT, mf, m1, m2k);
+                if constexpr (S::grad && yonly) grads_map_y<0>(g, gT, m1, tY[4*nY + jj + H]);
+                else if constexpr (S::grad) grads_map<0>(G, g, gT, mf, m1, m2k);
             }
             face_flux<0, S>(C, q, nc, nf, g, gT, P, pf);
             #pragma unroll
@@ -704,7 +707,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             if constexpr (MAP)
             {
                 const double m0 = tX[ii + H], mf = fY[cj];
-                if (yonly)
+                if constexpr (yonly)
                 {
                     #pragma unroll
                     for (int m = 0; m < NQ; ++m) nc[m] = tY[3*nY + cj - 1 - l + m + H];
@@ -720,7 +723,8 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
                     }
                     nf = nrm_at(mf, jac_at(m0, mf, m2k));
                 }
-                if constexpr (S::grad) grads_map<1>(G, g, gT, mf, m2k, m0);
+                if constexpr (S::grad && yonly) grads_map_y<1>(g, gT, mf, fY[2*nYf + cj]);
+                else if constexpr (S::grad) grads_map<1>(G, g, gT, mf, m2k, m0);
             }
             face_flux<1, S>(C, q, nc, nf, g, gT, P, pf);
             #pragma unroll
@@ -770,7 +774,8 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
             if constexpr (S::grad)
             {
                 tile_grads_z<S>(rz, rp, py, 3*pos, c0, c1, ix, iy, iz, g, gT);
-                if constexpr (MAP) grads_map<2>(G, g, gT, mf, m0i, m1j);
+                if constexpr (yonly) grads_map_y<2>(g, gT, m1j, tY[4*nY + j + H]);
+            else if constexpr (MAP) grads_map<2>(G, g, gT, mf, m0i, m1j);
             }
             if constexpr (S::wide)
             {
@@ -933,10 +938,13 @@ void launch_tile(const Grid& g, const double* prims, double* rhs, const spd_flux
     C.wi = p.wi; C.wj = p.wj; C.tx = p.tx; C.ty = p.ty; C.zs = p.zs;
     const dim3 grid((unsigned)(p.tx*p.ty*p.zs*G.nblk)), block((unsigned)p.nt);
     const int inc = increment ? 1 : 0;
-    if (map)
-        hipLaunchKernelGGL((k_flux_div_spec_tile<S, true>), grid, block, p.lds, s, G, prims, rhs, C, inc);
-    else
-        hipLaunchKernelGGL((k_flux_div_spec_tile<S, false>), grid, block, p.lds, s, G, prims, rhs, C, inc);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, p.lds, s, G, prims, rhs, C, inc); };
+    switch (map_variant(G))
+    {
+        case 0: go(k_flux_div_spec_tile<S, 0>); break;
+        case 1: go(k_flux_div_spec_tile<S, 1>); break;
+        case 2: go(k_flux_div_spec_tile<S, 2>); break;
+    }
     SPD_LAUNCH_CHECK();
 }
 

@@ -197,6 +197,14 @@ __device__ inline double map_deriv(const DevGeom& G, int d, double xi)
     return 1.0;
 }
 
+// The coordinates a face-once kernel is built for: 0 identity, 1 only y mapped
+// (its metrics then depend on the row alone), 2 any diagonal map
+inline int map_variant(const DevGeom& G)
+{
+    if (G.identity) return 0;
+    return G.map_kind[0] == SPD_MAP_IDENTITY && G.map_kind[2] == SPD_MAP_IDENTITY ? 1 : 2;
+}
+
 // The hardware hands workgroup w of a launch to XCD w mod 8.  A launch that
 // takes its work in XCD runs permutes its workgroup numbers with this map so
 // that each XCD takes one contiguous run of work items instead (XCD c: the
