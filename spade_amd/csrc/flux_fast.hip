@@ -28,6 +28,8 @@
 #include "spd_internal.hpp"
 #include "flux_face.hpp"
 #include "spd_stage.hpp"
+#include <algorithm>
+#include <cstdlib>
 
 namespace spd {
 namespace {
@@ -149,14 +151,14 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     __shared__ double sFx[5][16*17];      // x-face products, faces i = 0..16 of row j
     __shared__ double sFy[5][17*16];      // y-face products, faces j = 0..16 of column i
 
-    // zsplit 2 or 4: that many workgroups per block, each marching over its
-    // share of the planes [k0, k1) with its own window prologue (fewer, shorter tail rounds when
-    // the block count is not a multiple of the resident workgroups)
+    // zsplit workgroups per block, each marching over its share of the planes
+    // [k0, k1) with its own window prologue: small grids fill the device, and the
+    // tail rounds of a middling one are shorter
     // split: workgroups per block in the low byte, bit 8 set for XCD runs
     const int zsplit = split & 0xff;
     const int w = (split & 0x100) ? xcd_run_order(blockIdx.x, G.nblk*zsplit) : blockIdx.x;
     const int lb = w/zsplit, half = w - lb*zsplit;
-    const int k0 = half*(G.nc[2]/zsplit), k1 = k0 + G.nc[2]/zsplit;
+    const int k0 = G.nc[2]*half/zsplit, k1 = G.nc[2]*(half + 1)/zsplit;
     const int tid = threadIdx.x;
     const int i = tid & 15, j = tid >> 4;
     const double ix = G.inv_dx[3*lb + 0], iy = G.inv_dx[3*lb + 1], iz = G.inv_dx[3*lb + 2];
@@ -336,10 +338,10 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
         const double* sm = ring[0];
         const double* s0 = ring[1];
         const double* sp = ring[2];
-        const double* sk = sS[k & 1];
+        const double* sk = sS[(k - k0) & 1];
         // the cells of this column in planes k and k+1, from the window
         const CellV cur = cell_from_lds(sk, s0, pown);
-        const CellV nxt = cell_from_lds(sS[(k + 1) & 1], sp, pown);
+        const CellV nxt = cell_from_lds(sS[(k - k0 + 1) & 1], sp, pown);
         // the power law of the thread's three faces and, in waves 2 and 3, of
         // its block-boundary face
         double pw[4] = {1.0, 1.0, 1.0, 1.0};
@@ -576,7 +578,7 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
             // parity buffer of plane k; its raw registers take plane k+3
             double* s_new = ring[0];
             ring[0] = ring[1]; ring[1] = ring[2]; ring[2] = s_new;
-            double* t_new = sS[k & 1];
+            double* t_new = sS[(k - k0) & 1];
             if (INC)
             {
                 #pragma unroll
@@ -599,28 +601,23 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
     if (STG && A.push_ghosts) flush_x(G, A.push, A.qout, xs, lb, k1 - 1);   // after the last plane's closing barrier
 }
 
-// Workgroups per block (1, 2 or 4), each marching over an equal share of the
-// block's planes, chosen by rounds of resident workgroups (two per CU):
-// ceil(zs nblk / slots) rounds, each costing 1/zs of a block's march plus a
-// window prologue of about 0.1 of it.  A share must hold an even number of
-// planes.  SPD_FAST_ZSPLIT=1|2|4 forces the choice.
+// Workgroups per block, each marching over its share of the block's planes:
+// the least of rounds x (planes of a share + 0.65), with rounds the
+// workgroups over those resident at once (two per CU) and 0.65 planes the cost
+// of a share's prologue (256^3: 495, 514 and 550 us in 1, 2 and 4 shares).  64
+// blocks take 8 shares (one round of 512 workgroups; 64^3 ten steps 557 us, 669 in
+// 4 shares, 1076 in 2, 1935 whole), 576 blocks 4, 4096 blocks stay whole.
+// SPD_FAST_ZSPLIT=n forces the choice.
 int fast_zsplit(const Grid& g)
 {
-    const int nz = g.geom.nc[2];
-    auto ok = [&](int zs) { return nz % (2*zs) == 0; };
-    if (const char* e = getenv("SPD_FAST_ZSPLIT"))
-    {
-        const int zs = e[0] == '4' ? 4 : (e[0] == '2' ? 2 : 1);
-        return ok(zs) ? zs : 1;
-    }
+    const int nz = g.geom.nc[2], most = std::min(nz, 255);
+    if (const char* e = getenv("SPD_FAST_ZSPLIT")) return std::max(1, std::min(most, atoi(e)));
     const long slots = 2L*g.ctx->cus, nb = g.geom.nblk;
     int best = 1;
     double best_cost = 1e300;
-    for (int zs = 1; zs <= 4; zs *= 2)
+    for (int zs = 1; zs <= most; ++zs)
     {
-        if (!ok(zs)) continue;
-        const double rounds = (double)((zs*nb + slots - 1)/slots);
-        const double cost = rounds*(1.0/zs + (zs > 1 ? 0.1 : 0.0));
+        const double cost = (double)((zs*nb + slots - 1)/slots)*((nz + zs - 1)/zs + 0.65);
         if (cost < best_cost - 1e-9) { best_cost = cost; best = zs; }
     }
     return best;

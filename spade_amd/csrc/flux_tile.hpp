@@ -864,6 +864,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
 // of resident workgroups (as fast_zsplit), a share costing its planes plus
 // about two for its prologue: twelve 4 x 8 x 4 blocks run as 24 workgroups, 27
 // blocks of 32^3 as 432, 240 blocks of 24 x 20 x 12 as 480 of half a block each.
+constexpr double kTilePrologue = 0.65;
 struct TilePlan { int wi, wj, tx, ty, zs, nt; size_t lds; };
 
 inline TilePlan plan_tile(const DevGeom& G, int H, int SS, bool map, int cus)
@@ -895,11 +896,10 @@ inline TilePlan plan_tile(const DevGeom& G, int H, int SS, bool map, int cus)
     for (int zs = ceil_div(nz, 64); zs <= nz; ++zs)
     {
         const int share = ceil_div(nz, zs);
-        if (zs > 1 && share < 2 && nz > 2) break;
         const size_t lds = sizeof(double)*(size_t)TileLds(best.wi, best.wj, share, H, SS, map).total;
         const int per_cu = std::max(1, std::min((int)(160*1024/(lds + 2048)), 512/best.nt));
         const double rounds = std::ceil(tiles*zs/((double)per_cu*cus));
-        const double cost = rounds*(share + 2.0);
+        const double cost = rounds*(share + kTilePrologue);
         if (cost < best_cost - 1e-9) { best_cost = cost; best.zs = zs; best.lds = lds; }
     }
     return best;
