@@ -103,8 +103,7 @@ double* ensure_stage(Grid& g)
 void apply_bc(spd_integrator_s* it, double* a)
 {
     Grid& g = *it->q->a.grid;
-    for (int face = 0; face < 6; ++face)
-        if (it->bc.wall_mask & (1 << face)) launch_wall_fill(g, a ? a : it->q->a.d, face, it->bc.t_wall, g.ctx->stream);
+    launch_wall_fill(g, a ? a : it->q->a.d, it->bc.wall_mask, it->bc.t_wall, g.ctx->stream);
 }
 
 // The SSP-RK3 step runs as three fused flux + stage launches (ping-pong
@@ -427,7 +426,7 @@ int spd_boundary_fill_wall(spd_array_t arr, int face, double t_wall)
     {
         require(arr != nullptr, "null argument");
         require(face >= 0 && face < 6, "face must be 0..5");
-        launch_wall_fill(*arr->a.grid, arr->a.d, face, t_wall, arr->a.grid->ctx->stream);
+        launch_wall_fill(*arr->a.grid, arr->a.d, 1 << face, t_wall, arr->a.grid->ctx->stream);
     });
 }
 

@@ -33,9 +33,13 @@ k_exchange(DevGeom G, const int* __restrict__ nbr, double* __restrict__ a, int x
     exchange_item(G, nbr, a, lb, part*blockDim.x + threadIdx.x);
 }
 
+// Faces of axis idir in pms (bit 0 min, bit 1 max), blockIdx.z counting them:
+// the two faces of an axis neither read nor write each other's ghosts, so they
+// go in one launch
 __global__ void __launch_bounds__(256)
-k_wall_fill(DevGeom G, double* __restrict__ a, int idir, int pm, double t_wall)
+k_wall_fill(DevGeom G, double* __restrict__ a, int idir, int pms, double t_wall)
 {
+    const int pm = pms == 3 ? (int)blockIdx.z : pms >> 1;
     // blockIdx.y enumerates the blocks on the face: (b[d1], b[d2]), d1 < d2 the other axes
     const int d1 = idir == 0 ? 1 : 0, d2 = idir == 2 ? 1 : 2;
     int b[3];
@@ -294,17 +298,21 @@ void launch_exchange(const Grid& g, double* a, hipStream_t s)
     SPD_LAUNCH_CHECK();
 }
 
-void launch_wall_fill(const Grid& g, double* a, int face, double t_wall, hipStream_t s)
+void launch_wall_fill(const Grid& g, double* a, int face_mask, double t_wall, hipStream_t s)
 {
     const DevGeom& G = g.geom;
-    const int idir = face/2, pm = face % 2;
-    int ext[3] = {G.N[0], G.N[1], G.N[2]};
-    ext[idir] = G.ng;
-    const int n = ext[0]*ext[1]*ext[2];
-    const int d1 = idir == 0 ? 1 : 0, d2 = idir == 2 ? 1 : 2;
-    const int face_blocks = G.nb[d1]*G.nb[d2];
-    hipLaunchKernelGGL(k_wall_fill, dim3((n + 255)/256, face_blocks), dim3(256), 0, s, G, a, idir, pm, t_wall);
-    SPD_LAUNCH_CHECK();
+    for (int idir = 0; idir < 3; ++idir)
+    {
+        const int pms = (face_mask >> (2*idir)) & 3;
+        if (!pms) continue;
+        int ext[3] = {G.N[0], G.N[1], G.N[2]};
+        ext[idir] = G.ng;
+        const int n = ext[0]*ext[1]*ext[2];
+        const int d1 = idir == 0 ? 1 : 0, d2 = idir == 2 ? 1 : 2;
+        hipLaunchKernelGGL(k_wall_fill, dim3((n + 255)/256, G.nb[d1]*G.nb[d2], pms == 3 ? 2 : 1), dim3(256), 0, s,
+                           G, a, idir, pms, t_wall);
+        SPD_LAUNCH_CHECK();
+    }
 }
 
 // grid of one boundary face: ghost cells per face block x face blocks

@@ -68,8 +68,9 @@ void check_table(const spd_rk_table& tb)
 void set_ratio(spd_ratio& r, long n, long d) { r.num = n; r.den = d; }
 
 // The boundary of a stage: the caller's callback, else the exchange and the
-// isothermal walls of the descriptor
-void stage_bc(spd_integrator_s* it, spd_array_s* sol)
+// isothermal walls of the descriptor (exchanged: the stage launch has already
+// written the ghosts an exchange would copy)
+void stage_bc(spd_integrator_s* it, spd_array_s* sol, bool exchanged = false)
 {
     if (it->bcfn)
     {
@@ -77,10 +78,8 @@ void stage_bc(spd_integrator_s* it, spd_array_s* sol)
         return;
     }
     Grid& g = *sol->a.grid;
-    launch_exchange(g, sol->a.d, g.ctx->stream);
-    if (it->has_walls)
-        for (int face = 0; face < 6; ++face)
-            if (it->bc.wall_mask & (1 << face)) launch_wall_fill(g, sol->a.d, face, it->bc.t_wall, g.ctx->stream);
+    if (!exchanged) launch_exchange(g, sol->a.d, g.ctx->stream);
+    if (it->has_walls) launch_wall_fill(g, sol->a.d, it->bc.wall_mask, it->bc.t_wall, g.ctx->stream);
 }
 
 void stage_rhs(spd_integrator_s* it, spd_array_s* r, spd_array_s* sol)
@@ -95,11 +94,11 @@ void stage_rhs(spd_integrator_s* it, spd_array_s* r, spd_array_s* sol)
 
 // Evaluate residual i at t + c_i dt (the axis time moves there and back, as
 // axis.time() += time_coeff*dt; ...; axis.time() -= time_coeff*dt)
-void eval_stage(spd_integrator_s* it, int i, spd_array_s* sol, bool with_bc)
+void eval_stage(spd_integrator_s* it, int i, spd_array_s* sol, bool with_bc, bool exchanged = false)
 {
     const double tc = ratio_value(it->table.c[i].num, it->table.c[i].den);
     it->t += tc*it->dt;
-    if (with_bc) stage_bc(it, sol);
+    if (with_bc) stage_bc(it, sol, exchanged);
     stage_rhs(it, it->res[i], sol);
     it->t -= tc*it->dt;
 }
@@ -117,6 +116,7 @@ void advance_generic(spd_integrator_s* it)
     if (it->trans == SPD_TRANS_PRIM_CONS)
     {
         // transform-aware advance (advance.h:233-280)
+        const bool push = !it->bcfn;
         auto advance_to = [&](int prev, int curr)
         {
             const double* rr[SPD_RK_MAX_STAGES];
@@ -126,19 +126,19 @@ void advance_generic(spd_integrator_s* it)
                 rr[j] = it->res[j]->a.d;
                 coef[j] = row_diff(tb, curr, prev, j)*dt;   // zero entries are skipped by the kernel
             }
-            // the ghosts are left to the boundary step: with the caller's own
-            // bc the exchange may not be what follows
-            launch_rk_transform_stage(g, q->a.d, rr, coef, S, it->gamma, it->R, st, false);
+            // with the caller's own bc the exchange may not be what follows, so
+            // the ghosts are left to it
+            launch_rk_transform_stage(g, q->a.d, rr, coef, S, it->gamma, it->R, st, push);
         };
         eval_stage(it, 0, q, false);
         for (int i = 1; i < S; ++i)
         {
             advance_to(i - 1, i);
-            eval_stage(it, i, q, true);
+            eval_stage(it, i, q, true, push);
         }
         advance_to(S - 1, S);
         it->t += dt;
-        stage_bc(it, q);
+        stage_bc(it, q, push);
         return;
     }
     // generic advance with the identity transform (advance.h:107-230)
