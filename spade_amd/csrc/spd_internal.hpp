@@ -4,6 +4,7 @@
 #include <string>
 #include <vector>
 #include <cstdint>
+#include <mutex>
 #include "../../include/spade_amd.h"
 
 namespace spd {
@@ -56,6 +57,14 @@ struct Ctx
     double* h_io[2] = {nullptr, nullptr};
     size_t h_io_doubles = 0;
     hipEvent_t io_ev[2] = {nullptr, nullptr};
+    // pinned slots of large downloads, one per copying thread (api.cpp),
+    // allocated on first use and freed with the context; the mutex is held for
+    // a whole download
+    static constexpr int kCopyThreads = 4;
+    static constexpr size_t kCopySlot = 4u << 20;
+    std::mutex copy_mu;
+    char* copy_slot = nullptr;            // kCopyThreads slots of kCopySlot bytes
+    hipEvent_t copy_ev[kCopyThreads] = {};
 };
 
 struct Grid

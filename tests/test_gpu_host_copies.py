@@ -1,0 +1,45 @@
+"""Host arrays large enough to move in pieces by several threads: odd sizes
+come back as they went, also from two host threads sharing one context."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _round_trips(sa, blocks, cells, seed, n=1):
+    g = sa.CartesianGrid(cells, blocks, ((0.0, 1.0),) * 3)
+    a = sa.GridArray(g)
+    rng = np.random.default_rng(seed)
+    for _ in range(n):
+        host = rng.standard_normal(g.host_shape)
+        a.upload(host)
+        if not np.array_equal(a.download(), host):
+            return False
+    return True
+
+
+@pytest.mark.parametrize("blocks, cells", [((1, 1, 7), (16, 16, 16)), ((3, 2, 2), (17, 19, 33)),
+                                           ((5, 5, 7), (16, 16, 16)), ((1, 1, 1), (120, 11, 90))])
+def test_round_trip(blocks, cells):
+    import spade_amd as sa
+    sa.load()
+    print(blocks, cells, flush=True)
+    assert _round_trips(sa, blocks, cells, 3)
+
+
+def test_two_threads_one_context():
+    import spade_amd as sa
+    sa.load()
+    sa.default_context()
+    ok = [False, False]
+
+    def go(t):
+        ok[t] = _round_trips(sa, (4, 4, 2 + t), (16, 16, 16), t, n=4)
+    threads = [threading.Thread(target=go, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert ok == [True, True]
