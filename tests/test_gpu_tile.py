@@ -88,3 +88,35 @@ def test_planes_outside_the_series_equal_per_cell(name):
 
 def test_one_ghost_layer_equal_per_cell():
     _compare((7, 10, 5), (1, 2, 1), FLUXES["keep2_visc"], ng=1)
+
+
+@pytest.mark.parametrize("name", ["weno_visc", "fweno_visc"])
+@pytest.mark.parametrize("p, jump", [(1e-12, 1.0), (1.0, 0.0), (1.0, 1e6), (1e55, 1.0), (1.0, np.inf)],
+                         ids=["faint", "uniform", "shock", "huge", "infinite"])
+def test_weno_quotients_equal_per_cell(p, jump, name):
+    """The smooth weights' own quotients over the range of their squares (1e-32
+    for equal fluxes, about 1e220 for "huge") and through an infinite cell."""
+    import spade_amd as sa
+    g = sa.CartesianGrid((19, 18, 5), (1, 2, 1), ((0.0, 2.0), (-1.0, 1.0), (0.0, 1.5)), num_exch=2)
+    q = np.random.default_rng(4).standard_normal(g.host_shape)
+    q *= 0.0 if jump == 0.0 else 1.0
+    q[..., 0] = p * (1.0 + 0.3 * np.tanh(q[..., 0]))
+    q[..., 1] = 1.1 * (1.0 + 0.005 * q[..., 1])
+    q[..., 2:] = 0.3 + 0.2 * q[..., 2:]
+    if jump:
+        q[0, 6, 9:, :, 0] *= jump
+    arr = sa.GridArray(g).upload(q)
+    flux = RawFlux(FLUXES[name], GAMMA, R)
+    out = []
+    for generic in (False, True):
+        if generic:
+            os.environ["SPD_DISABLE_SPEC"] = "1"
+        try:
+            rhs = sa.GridArray(g)
+            sa.flux_div(arr, rhs, flux)
+            out.append(rhs.download())
+        finally:
+            os.environ.pop("SPD_DISABLE_SPEC", None)
+    print(name, p, jump, np.isnan(out[0]).sum(), flush=True)
+    assert np.array_equal(out[0], out[1], equal_nan=True)
+    assert np.isfinite(out[0]).all() == np.isfinite(jump)
