@@ -458,6 +458,16 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     constexpr double sc = 1.0/S::scale;
     constexpr int Y = 2*H + 1;                // (z tables start at plane k0 - H)
     const int tid = threadIdx.x;
+    // thread number of the halo columns and the closing faces.  Wide stencils
+    // and WALE, whose waves with a fourth face bind the SIMD they run on, take
+    // closing faces in waves 1 and 3 and halo columns in 0 and 2: the two
+    // workgroups of a CU are placed one SIMD on from each other, so each SIMD
+    // then holds one such wave, where of waves 2 and 3 one SIMD held two
+    // ({WENO, viscous} 128^3 217 -> 212 us, {KEEP4, WALE} 96^3 91.2 -> 88.3).
+    // The lighter KEEP2 kernels wait for memory instead and keep waves 2 and
+    // 3 (67.4 us against 68.2 on 24x20x12 blocks).
+    constexpr bool heavy = S::wide || S::wale;
+    const int rt = heavy && blockDim.x == 256 ? (tid & 63) | ((tid & 64) << 1) | ((tid & 128) >> 1) : tid;
 
     // work item: block, share of planes, tile, neighbours next to each other on an XCD
     int w = xcd_run_order(blockIdx.x, gridDim.x);
@@ -524,25 +534,25 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     const int own = (int)stored_offset(G, i0 + i, j0 + j, 0);
     const int nhalo = 2*H*(wi + wj) + 4;
     int hpos = -1, hi = 0, hj = 0;
-    const bool hcorner = tid >= nhalo - 4;
-    if (tid < 2*H*wj)
+    const bool hcorner = rt >= nhalo - 4;
+    if (rt < 2*H*wj)
     {
-        const int a = tid/wj, lay = a >> 1;
-        hj = tid - a*wj;
+        const int a = rt/wj, lay = a >> 1;
+        hj = rt - a*wj;
         hi = (a & 1) ? wi + lay : -1 - lay;
     }
-    else if (tid < nhalo - 4)
+    else if (rt < nhalo - 4)
     {
-        const int t = tid - 2*H*wj, a = t/wi, lay = a >> 1;
+        const int t = rt - 2*H*wj, a = t/wi, lay = a >> 1;
         hi = t - a*wi;
         hj = (a & 1) ? wj + lay : -1 - lay;
     }
-    else if (tid < nhalo)
+    else if (rt < nhalo)
     {
-        const int c = tid - (nhalo - 4);
+        const int c = rt - (nhalo - 4);
         hi = (c & 1) ? wi : -1; hj = (c & 2) ? wj : -1;
     }
-    if (tid < nhalo) hpos = (hj + H)*PX + (hi + H);
+    if (rt < nhalo) hpos = (hj + H)*PX + (hi + H);
     const int hoff = (int)stored_offset(G, i0 + hi, j0 + hj, 0);
     const int hstr = (i0 + hi >= 0 && i0 + hi < G.nc[0]) ? plane : xplane;
     auto load = [&](int off) -> Raw5
@@ -651,10 +661,10 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
     // the closing faces of the tile are evaluated by lanes of the last two
     // waves, or all by the last one where it has no columns of its own
     const int nw = blockDim.x >> 6;
-    const int by = tid - (nw - 1)*64;
-    const int bx = wi*wj <= (nw - 1)*64 ? by : tid - max(nw - 2, 0)*64;
+    const int by = rt - (nw - 1)*64;
+    const int bx = wi*wj <= (nw - 1)*64 ? by : rt - max(nw - 2, 0)*64;
 
-    const bool closing = __builtin_amdgcn_readfirstlane(tid) >= 64*max(nw - 2, 0);   // a wave with closing faces
+    const bool closing = __builtin_amdgcn_readfirstlane(rt) >= 64*max(nw - 2, 0);   // a wave with closing faces
 
     for (int k = k0; k < k1; ++k)
     {
