@@ -764,6 +764,7 @@ int spd_batch_set_shape(spd_batch_t b, int grid, int interleaved)
     {
         require(b != nullptr, "null argument");
         require(grid >= 1 && grid <= 65536, "grid must be in 1..65536");
+        b->b->fix_shape();
         b->b->grid = grid;
         if (b->b->order_interleaved != (interleaved != 0)) { b->b->order_interleaved = interleaved != 0; b->b->worklist_dirty = true; }
     });
@@ -777,6 +778,7 @@ int spd_batch_set_kernel_shape(spd_batch_t b, int rows, int prefetch, int occupa
         require(rows == 16 || rows == 8, "rows must be 16 or 8");
         require(prefetch == 1 || prefetch == 2, "prefetch must be 1 or 2");
         require(occupancy == 2 || occupancy == 3, "occupancy must be 2 or 3");
+        b->b->fix_shape();
         b->b->variant = spd::batch_variant(rows, prefetch, occupancy);
     });
 }

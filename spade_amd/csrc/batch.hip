@@ -17,7 +17,7 @@
 //     with D(U) = -div u evaluated per cell in FP64 from FP64 velocities, and
 //     the constant p_ref n momentum flux cancels exactly;
 //   * kinetic energy and enstrophy of the stage-1 input state are summed per
-//     block (fixed-order tree) for the per-case diagnostics history.
+//     half block in a fixed order for the per-case diagnostics history.
 #include "spd_internal.hpp"
 #include "batch.hpp"
 #include <cmath>
@@ -187,10 +187,12 @@ __device__ inline CaseParams uniform_params(const CaseParams& c)
 //        56-172 bytes per lane spilled, 2: up to 256 VGPRs without); a
 //        256-thread workgroup holds 48.5 KB of LDS and a 128-thread one
 //        26.5 KB, so three or six of them fit a CU.
+//   zs   workgroups along a block's planes (1, 2 or 4, an argument), each
+//        marching over its share with a window prologue of its own.
 // Every shape evaluates the same expressions in the same order, and the
-// per-block diagnostics are summed over the same two half-block trees (rows
-// 0-7 and 8-15, 128 leaves each, added on the host), so all shapes give the
-// same bits.
+// per-block diagnostics are summed over the same units of 4 rows by 4 planes
+// (kBatchParts of them, one wave each, in a fixed tree; added in order by the
+// next stage), so all shapes give the same bits.
 template <int TJ> struct Tile
 {
     static constexpr int NT = 16*TJ;                     // threads
@@ -207,8 +209,10 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
         double alpha, double beta, int flags)
 {
     using T = Tile<TJ>;
-    // flags: bit 0 per-block diagnostics, bit 1 work items in XCD runs
+    // flags: bit 0 sum the diagnostics of each unit of rows and planes, bit 1
+    // work items in XCD runs, bit 2 add the units up; from bit 8 zs
     const bool want_diag = flags & 1;
+    const int zs = flags >> 8;
     constexpr int HP = T::HP, NTILE = 16/TJ;
     __shared__ float  sU[3][3*HP];        // u, v, w (f32) of planes k-1, k, k+1
     __shared__ float  sS[2][4*HP];        // p', T', rho', e' of planes k, k+1 (parity)
@@ -217,12 +221,6 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
     // read them, which is exact, so every shape sums the same doubles
     __shared__ alignas(16) float sFx[5][TJ*17];
     __shared__ float sFy[5][(TJ + 1)*16];
-    // the per-block diagnostics tree reuses the x-face buffer after the
-    // k-march (the march's last barrier has passed, and the next work item
-    // writes face fluxes only after its prologue barrier); the window plus
-    // the fluxes then fit three 256-thread or six 128-thread workgroups per CU
-    static_assert(sizeof(double)*2*T::NT <= sizeof(sFx), "diagnostics tree exceeds the x-face buffer");
-    double (*sRed)[T::NT] = reinterpret_cast<double (*)[T::NT]>(&sFx[0][0]);
 
     const int tid = threadIdx.x;
     const int i = tid & 15, j = tid >> 4;                // j: row within the tile
@@ -234,7 +232,8 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
     else if (tid < 2*TJ + 32) { hi = tid - 2*TJ - 16; hj = TJ; }
     else if (tid < T::NHALO)  { const int c = tid - 2*TJ - 32; hi = (c & 1) ? 16 : -1; hj = (c & 2) ? TJ : -1; }
     const int pown = lposb(i, j), phalo = lposb(hi, hj);
-    const int nitems = *B.nwork*NTILE;
+    const int per_slot = NTILE*zs;
+    const int nitems = *B.nwork*per_slot;
 
     // XCD runs: the workgroups on one XCD take consecutive work items of each
     // round (neighbour blocks of a case, in case-major order) instead of every
@@ -244,8 +243,18 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
     {
         // slot and case constants are the same for the whole workgroup: held
         // in scalar registers, not reloaded per lane inside the k-march
-        const int slot = __builtin_amdgcn_readfirstlane(B.worklist[w/NTILE]);
-        const int j0 = (w % NTILE)*TJ;                   // first row of the tile in the block
+        const int slot = __builtin_amdgcn_readfirstlane(B.worklist[w/per_slot]);
+        const int part = w % per_slot;
+        const int j0 = (part % NTILE)*TJ;                // first row of the tile in the block
+        const int k0 = 16/zs*(part/NTILE), k1 = k0 + 16/zs;   // its planes
+        if ((flags & 4) && part == 0 && tid < 4)
+        {
+            // the units of the stage before, {ke, enstrophy} per half block
+            const double* u = B.parts + (long long)slot*2*kBatchParts + (tid >> 1)*kBatchParts + (tid & 1);
+            double sum = 0.0;
+            for (int n = 0; n < kBatchParts/2; ++n) sum += u[2*n];
+            B.diag[((long long)(*B.step % B.hist_len)*B.max_slots + slot)*4 + tid] = sum;
+        }
         const CaseParams P = uniform_params(B.cases[__builtin_amdgcn_readfirstlane(B.slot_case[slot])]);
         const int* nb = B.nbr + 27*slot;
         const float ix = (float)P.ix, iy = (float)P.iy, iz = (float)P.iz;
@@ -295,34 +304,34 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
         // the plane's first barrier instead of a plane ahead, so that it is not
         // live across the face evaluation
         constexpr bool late_u0 = OCC == 3;
-        if (!late_u0) load_u0(0);
+        if (!late_u0) load_u0(k0);
 
-        // prologue: planes -1, 0, 1 resident, planes 2 .. 1 + PFB in flight.
+        // prologue: planes k0-1, k0, k0+1 resident, planes k0+2 .. k0+1+PFB in flight.
         // The own column's conserved state of planes k and k+1 stays in
         // registers (the stage input u_in); velocities of planes k, k+1 are in LDS.
-        const PrimD qprev = to_prim(P, load_col(own_slot, i, gj, -1));
-        Cons rcur = load_col(own_slot, i, gj, 0);
-        Cons rnxt = load_col(own_slot, i, gj, 1);
+        const PrimD qprev = to_prim(P, load_col(own_slot, i, gj, k0 - 1));
+        Cons rcur = load_col(own_slot, i, gj, k0);
+        Cons rnxt = load_col(own_slot, i, gj, k0 + 1);
         const PrimD qcur0 = to_prim(P, rcur), qnxt0 = to_prim(P, rnxt);
         CellF prev = to_f32(P, qprev), cur = to_f32(P, qcur0), nxt = to_f32(P, qnxt0);
         Cons nraw[PFB], hraw[PFB];
         #pragma unroll
-        for (int d = 0; d < PFB; ++d) { nraw[d] = load_col(own_slot, i, gj, 2 + d); hraw[d] = Cons{}; }
+        for (int d = 0; d < PFB; ++d) { nraw[d] = load_col(own_slot, i, gj, k0 + 2 + d); hraw[d] = Cons{}; }
         {
-            float* s = sU[slotk(-1)];
+            float* s = sU[slotk(k0 - 1)];
             s[pown] = prev.u; s[HP + pown] = prev.v; s[2*HP + pown] = prev.w;
         }
-        put(0, pown, qcur0, cur); put(1, pown, qnxt0, nxt);
+        put(k0, pown, qcur0, cur); put(k0 + 1, pown, qnxt0, nxt);
         if (has_halo)
         {
-            const CellF hp = to_f32(P, to_prim(P, load_col(halo_slot, hi, ghj, -1)));
-            float* s = sU[slotk(-1)];
+            const CellF hp = to_f32(P, to_prim(P, load_col(halo_slot, hi, ghj, k0 - 1)));
+            float* s = sU[slotk(k0 - 1)];
             s[phalo] = hp.u; s[HP + phalo] = hp.v; s[2*HP + phalo] = hp.w;
-            const PrimD h0 = to_prim(P, load_col(halo_slot, hi, ghj, 0)), h1 = to_prim(P, load_col(halo_slot, hi, ghj, 1));
-            put(0, phalo, h0, to_f32(P, h0));
-            put(1, phalo, h1, to_f32(P, h1));
+            const PrimD h0 = to_prim(P, load_col(halo_slot, hi, ghj, k0)), h1 = to_prim(P, load_col(halo_slot, hi, ghj, k0 + 1));
+            put(k0, phalo, h0, to_f32(P, h0));
+            put(k0 + 1, phalo, h1, to_f32(P, h1));
             #pragma unroll
-            for (int d = 0; d < PFB; ++d) hraw[d] = load_col(halo_slot, hi, ghj, 2 + d);
+            for (int d = 0; d < PFB; ++d) hraw[d] = load_col(halo_slot, hi, ghj, k0 + 2 + d);
         }
         double ke_acc = 0.0, en_acc = 0.0;
         double wprev_u = qprev.u, wprev_v = qprev.v, wprev_w = qprev.w;   // own column, plane k-1 (f64)
@@ -331,13 +340,13 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
         float zlo[5];                    // low z-face flux of the current plane (widened where used)
         {
             float g[3][3], gT, F[5];
-            gradsf_z<HP>(sU[slotk(-1)], sU[slotk(0)], pown, prev, cur, ix, iy, iz, g, gT);
+            gradsf_z<HP>(sU[slotk(k0 - 1)], sU[slotk(k0)], pown, prev, cur, ix, iy, iz, g, gT);
             face_f32<2, LAW>(P, prev, cur, g, gT, F);
             #pragma unroll
             for (int n = 0; n < 5; ++n) zlo[n] = F[n];
         }
 
-        for (int k = 0; k < 16; ++k)
+        for (int k = k0; k < k1; ++k)
         {
             const long long o = (long long)slot*5*4096 + (k*16 + gj)*16 + i;
             const float* sm = sU[slotk(k - 1)];
@@ -406,6 +415,22 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
                 const double uc = vk[pown], vc = vk[HP + pown], wc = vk[2*HP + pown];
                 ke_acc += 0.5*rcur.r*(uc*uc + vc*vc + wc*wc);
                 en_acc += 0.5*(ox*ox + oy*oy + oz*oz);
+                if ((k & 3) == 3)
+                {
+                    // a unit of 4 rows (this wave's) and 4 planes is complete
+                    #pragma unroll
+                    for (int d = 32; d > 0; d >>= 1)
+                    {
+                        ke_acc += __shfl_down(ke_acc, d);
+                        en_acc += __shfl_down(en_acc, d);
+                    }
+                    if ((tid & 63) == 0)
+                    {
+                        double* u = B.parts + (long long)slot*2*kBatchParts + 2*(((j0 >> 2) + (tid >> 6))*4 + (k >> 2));
+                        u[0] = ke_acc; u[1] = en_acc;
+                    }
+                    ke_acc = 0.0; en_acc = 0.0;
+                }
             }
             if (late_u0) load_u0(k);
             lds_barrier();
@@ -438,7 +463,7 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
 
             // advance the window
             wprev_u = vk[pown]; wprev_v = vk[HP + pown]; wprev_w = vk[2*HP + pown];
-            if (k + 1 < 16)
+            if (k + 1 < k1)
             {
                 if (!late_u0) load_u0(k + 1);
                 rcur = rnxt; rnxt = nraw[0]; cur = nxt;
@@ -447,34 +472,15 @@ k_stage(BatchDev B, const double* __restrict__ Qin, const double* __restrict__ Q
                 put(k + 2, pown, q2, nxt);
                 #pragma unroll
                 for (int d = 0; d + 1 < PFB; ++d) nraw[d] = nraw[d + 1];
-                if (k + 2 + PFB <= 16) nraw[PFB - 1] = load_col(own_slot, i, gj, k + 2 + PFB);
+                if (k + 2 + PFB <= k1) nraw[PFB - 1] = load_col(own_slot, i, gj, k + 2 + PFB);
                 if (has_halo)
                 {
                     const PrimD hq = to_prim(P, hraw[0]);
                     put(k + 2, phalo, hq, to_f32(P, hq));
                     #pragma unroll
                     for (int d = 0; d + 1 < PFB; ++d) hraw[d] = hraw[d + 1];
-                    if (k + 2 + PFB <= 16) hraw[PFB - 1] = load_col(halo_slot, hi, ghj, k + 2 + PFB);
+                    if (k + 2 + PFB <= k1) hraw[PFB - 1] = load_col(halo_slot, hi, ghj, k + 2 + PFB);
                 }
-            }
-            lds_barrier();
-        }
-        if (want_diag)
-        {
-            // one 128-leaf tree per half block (rows 0-7, 8-15), the same in every shape
-            sRed[0][tid] = ke_acc; sRed[1][tid] = en_acc;
-            lds_barrier();
-            for (int s = 64; s > 0; s >>= 1)
-            {
-                if ((tid & 127) < s) { sRed[0][tid] += sRed[0][tid + s]; sRed[1][tid] += sRed[1][tid + s]; }
-                lds_barrier();
-            }
-            if ((tid & 127) == 0)
-            {
-                const int half = (j0 + j) >> 3;
-                const int h = *B.step % B.hist_len;
-                B.diag[(((long long)h*B.max_slots + slot)*2 + half)*2 + 0] = sRed[0][tid];
-                B.diag[(((long long)h*B.max_slots + slot)*2 + half)*2 + 1] = sRed[1][tid];
             }
             lds_barrier();
         }
@@ -541,26 +547,26 @@ namespace {
 // shape variant v: PFB = 1 + (v & 1), OCC = (v & 2) ? 2 : 3, TJ = (v & 4) ? 8 : 16
 template <int LAW, bool HAS_U0, int TJ, int PFB, int OCC>
 void launch_one(int grid, hipStream_t s, const BatchDev& B, const double* Qin, const double* Q0, double* Qout,
-                double alpha, double beta, int want_diag)
+                double alpha, double beta, int flags)
 {
     hipLaunchKernelGGL((k_stage<LAW, HAS_U0, TJ, PFB, OCC>), dim3(grid), dim3(16*TJ), 0, s,
-                       B, Qin, Q0, Qout, alpha, beta, want_diag);
+                       B, Qin, Q0, Qout, alpha, beta, flags);
 }
 
 template <int LAW, bool HAS_U0>
 void launch_shape(int v, const BatchDev& B, const double* Qin, const double* Q0, double* Qout,
-                  double alpha, double beta, int want_diag, int grid, hipStream_t s)
+                  double alpha, double beta, int flags, int grid, hipStream_t s)
 {
     switch (v)
     {
-    case 0:  launch_one<LAW, HAS_U0, 16, 1, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 1:  launch_one<LAW, HAS_U0, 16, 2, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 2:  launch_one<LAW, HAS_U0, 16, 1, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 3:  launch_one<LAW, HAS_U0, 16, 2, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 4:  launch_one<LAW, HAS_U0, 8, 1, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 5:  launch_one<LAW, HAS_U0, 8, 2, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    case 6:  launch_one<LAW, HAS_U0, 8, 1, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
-    default: launch_one<LAW, HAS_U0, 8, 2, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, want_diag); break;
+    case 0:  launch_one<LAW, HAS_U0, 16, 1, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 1:  launch_one<LAW, HAS_U0, 16, 2, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 2:  launch_one<LAW, HAS_U0, 16, 1, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 3:  launch_one<LAW, HAS_U0, 16, 2, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 4:  launch_one<LAW, HAS_U0, 8, 1, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 5:  launch_one<LAW, HAS_U0, 8, 2, 3>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    case 6:  launch_one<LAW, HAS_U0, 8, 1, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
+    default: launch_one<LAW, HAS_U0, 8, 2, 2>(grid, s, B, Qin, Q0, Qout, alpha, beta, flags); break;
     }
 }
 
@@ -602,21 +608,23 @@ static int batch_xcd_runs()
 }
 
 void launch_batch_stage(const BatchDev& B, int law, int variant, const double* Qin, const double* Q0, double* Qout,
-                        double alpha, double beta, int want_diag, int grid, hipStream_t s)
+                        double alpha, double beta, int stage, int zs, int grid, hipStream_t s)
 {
     if (variant < 0 || variant >= kBatchShapeVariants) throw ArgError{"batch kernel shape variant out of range"};
-    want_diag = (want_diag ? 1 : 0) | (batch_xcd_runs() ? 2 : 0);
+    if (zs != 1 && zs != 2 && zs != 4) throw ArgError{"batch plane shares out of range"};
+    // the first stage sums the diagnostics of its input, the second adds them up
+    const int flags = (stage == 1 ? 1 : stage == 2 ? 4 : 0) | (batch_xcd_runs() ? 2 : 0) | zs << 8;
     // stage 1 of the Shu-Osher form (alpha = 0) reads no u0
     const bool u0 = alpha != 0.0;
     if (law == SPD_LAW_POWER)
     {
-        if (u0) launch_shape<SPD_LAW_POWER, true>(variant, B, Qin, Q0, Qout, alpha, beta, want_diag, grid, s);
-        else    launch_shape<SPD_LAW_POWER, false>(variant, B, Qin, Q0, Qout, alpha, beta, want_diag, grid, s);
+        if (u0) launch_shape<SPD_LAW_POWER, true>(variant, B, Qin, Q0, Qout, alpha, beta, flags, grid, s);
+        else    launch_shape<SPD_LAW_POWER, false>(variant, B, Qin, Q0, Qout, alpha, beta, flags, grid, s);
     }
     else
     {
-        if (u0) launch_shape<SPD_LAW_CONST, true>(variant, B, Qin, Q0, Qout, alpha, beta, want_diag, grid, s);
-        else    launch_shape<SPD_LAW_CONST, false>(variant, B, Qin, Q0, Qout, alpha, beta, want_diag, grid, s);
+        if (u0) launch_shape<SPD_LAW_CONST, true>(variant, B, Qin, Q0, Qout, alpha, beta, flags, grid, s);
+        else    launch_shape<SPD_LAW_CONST, false>(variant, B, Qin, Q0, Qout, alpha, beta, flags, grid, s);
     }
     SPD_LAUNCH_CHECK();
 }

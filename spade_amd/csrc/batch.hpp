@@ -26,6 +26,10 @@ struct CaseIC
     double xc, yc, beta, dT;                 // vortex centre, strength, temperature dip
 };
 
+// Units of 4 rows by 4 planes of a block whose diagnostics one wave sums, in
+// the order row group, plane group (the first half of them: rows 0-7)
+constexpr int kBatchParts = 16;
+
 struct BatchDev
 {
     const int* worklist;                     // slots to advance
@@ -34,6 +38,7 @@ struct BatchDev
     const int* nbr;                          // [27*slot + e] neighbour slot (periodic within case)
     const CaseParams* cases;
     double* diag;                            // [hist][slot][half][2]: kinetic energy, enstrophy sums per half block
+    double* parts;                           // [slot][kBatchParts][2]: the same sums per 4 rows x 4 planes
     int* step;                               // device step counter (history row)
     int max_slots;
     int hist_len;
@@ -52,8 +57,9 @@ inline int batch_variant(int rows, int prefetch, int occupancy)
     return (prefetch - 1) | (occupancy == 2 ? 2 : 0) | (rows == 8 ? 4 : 0);
 }
 
+// stage: 1..3 of a step; zs: workgroups along a block's planes (1, 2 or 4)
 void launch_batch_stage(const BatchDev& B, int law, int variant, const double* Qin, const double* Q0, double* Qout,
-                        double alpha, double beta, int want_diag, int grid, hipStream_t s);
+                        double alpha, double beta, int stage, int zs, int grid, hipStream_t s);
 void launch_batch_step_count(const BatchDev& B, hipStream_t s);
 // Workgroups of the stage kernel (for law and shape variant) resident per CU
 // at once: the default persistent grid is this many per CU

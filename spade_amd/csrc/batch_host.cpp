@@ -38,6 +38,7 @@ Batch::Batch(Ctx* c, long long budget_bytes, int law_in, int hist) : ctx(c), law
     SPD_HIP(hipMalloc((void**)&d_small, sizeof(int)*64));
     SPD_HIP(hipMalloc((void**)&d_cases, sizeof(CaseParams)*(size_t)max_cases));
     SPD_HIP(hipMalloc((void**)&d_diag, sizeof(double)*4*(size_t)hist_len*max_slots));
+    SPD_HIP(hipMalloc((void**)&d_parts, sizeof(double)*2*kBatchParts*(size_t)max_slots));
     SPD_HIP(hipMalloc((void**)&d_init_slots, sizeof(int)*29*(size_t)max_slots));
     SPD_HIP(hipMemsetAsync(d_small, 0, sizeof(int)*64, ctx->stream));
     SPD_HIP(hipMemsetAsync(d_diag, 0, sizeof(double)*4*(size_t)hist_len*max_slots, ctx->stream));
@@ -50,17 +51,18 @@ Batch::Batch(Ctx* c, long long budget_bytes, int law_in, int hist) : ctx(c), law
     int cus = 0;
     SPD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     num_cu = std::max(1, cus);
-    // as many persistent workgroups as fit at once (spd_batch_tune may pick another)
-    grid = batch_stage_blocks_per_cu(law, variant)*num_cu;
-    dev = BatchDev{d_worklist, d_small + 0, d_slot_case, d_nbr, d_cases, d_diag, d_small + 1, max_slots, hist_len};
+    // as many persistent workgroups as fit at once
+    for (int v = 0; v < kBatchShapeVariants; ++v) resident[v] = batch_stage_blocks_per_cu(law, v);
+    grid = resident[variant]*num_cu;
+    dev = BatchDev{d_worklist, d_small + 0, d_slot_case, d_nbr, d_cases, d_diag, d_parts, d_small + 1, max_slots, hist_len};
 }
 
 Batch::~Batch()
 {
-    if (gexec) (void)hipGraphExecDestroy(gexec);
+    for (auto& v : gexec) for (auto g : v) if (g) (void)hipGraphExecDestroy(g);
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipFree(Q[0]); (void)hipFree(d_worklist); (void)hipFree(d_slot_case); (void)hipFree(d_nbr);
-    (void)hipFree(d_small); (void)hipFree(d_cases); (void)hipFree(d_diag); (void)hipFree(d_init_slots);
+    (void)hipFree(d_small); (void)hipFree(d_cases); (void)hipFree(d_diag); (void)hipFree(d_parts); (void)hipFree(d_init_slots);
 }
 
 long long Batch::footprint(const spd_case_desc& d)
@@ -217,27 +219,82 @@ void Batch::upload_worklist()
     worklist_dirty = false;
 }
 
+// Workgroups along the planes of a block, as log2: the least of rounds x
+// (planes of a share + 0.6), with rounds the work items over the workgroups
+// that run at once and 0.6 planes the cost of a share's window prologue (1420
+// blocks, 1.9 to 7.4 rounds: four steps take 1945, 2016 and 2150 us in 1, 2
+// and 4 shares).  168 blocks in 4 shares 400 us, 938 whole; 322 in 2 shares 600,
+// 952 whole; 3201 in 2 shares, whose last round is fuller, 4355, 4502 whole.
+int Batch::plane_shares(int v, int g, double* cost) const
+{
+    const long items = (long)nwork*(16/batch_variant_rows(v));
+    const long slots = std::max(1, std::min(g, resident[v]*num_cu));
+    int best = 0;
+    double best_cost = 1e300;
+    for (int z = 0; z < 3; ++z)
+    {
+        const double c = (double)(((items << z) + slots - 1)/slots)*((16 >> z) + 0.6);
+        if (c < best_cost - 1e-9) { best_cost = c; best = z; }
+    }
+    if (cost) *cost = best_cost;
+    return best;
+}
+
+// The shape for the work list where the caller set none: half-block workgroups
+// (1 to 2 % ahead of whole-block ones from 1420 blocks on, level below), with
+// registers for two waves per SIMD where those take fewer planes in all.  A
+// plane then costs 0.82 (168 and 322 blocks in one round 917 -> 757 and 933 ->
+// 768 us) but fewer workgroups run at once: 24 blocks take 306 us with two
+// and 370 with three, 322 blocks 690 and 600, 3201 blocks 4600 and 4315.
+void Batch::choose_shape()
+{
+    const int three = batch_variant(8, 1, 3), two = batch_variant(8, 1, 2);
+    double c3, c2;
+    plane_shares(three, resident[three]*num_cu, &c3);
+    plane_shares(two, resident[two]*num_cu, &c2);
+    variant = 0.82*c2 < c3 ? two : three;
+    grid = resident[variant]*num_cu;
+}
+
+// The caller's or the tuner's choice starts from whole-block workgroups
+void Batch::fix_shape()
+{
+    if (shape_set) return;
+    shape_set = true;
+    variant = 0;
+    grid = resident[0]*num_cu;
+}
+
 void Batch::enqueue_step(hipStream_t s)
 {
     // Shu-Osher SSP-RK3: u1 = u0 + dt L(u0); u2 = 3/4 u0 + 1/4 (u1 + dt L(u1));
     // u3 = 1/3 u0 + 2/3 (u2 + dt L(u2)).  Q0 -> Q1 -> Q2 -> Q0.
-    launch_batch_stage(dev, law, variant, Q[0], Q[0], Q[1], 0.0, 1.0, 1, grid, s);
-    launch_batch_stage(dev, law, variant, Q[1], Q[0], Q[2], 0.75, 0.25, 0, grid, s);
-    launch_batch_stage(dev, law, variant, Q[2], Q[0], Q[0], 1.0/3.0, 2.0/3.0, 0, grid, s);
+    const int zs = 1 << plane_shares(variant, grid);
+    launch_batch_stage(dev, law, variant, Q[0], Q[0], Q[1], 0.0, 1.0, 1, zs, grid, s);
+    launch_batch_stage(dev, law, variant, Q[1], Q[0], Q[2], 0.75, 0.25, 2, zs, grid, s);
+    launch_batch_stage(dev, law, variant, Q[2], Q[0], Q[0], 1.0/3.0, 2.0/3.0, 3, zs, grid, s);
     launch_batch_step_count(dev, s);
 }
 
-void Batch::build_graph()
+// The graph of one step in the shape in use, recorded on its first use
+hipGraphExec_t Batch::step_graph()
 {
-    if (gexec) { SPD_HIP(hipGraphExecDestroy(gexec)); gexec = nullptr; }
-    hipGraph_t g = nullptr;
-    SPD_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_step(ctx->stream);
-    SPD_HIP(hipStreamEndCapture(ctx->stream, &g));
-    SPD_HIP(hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0));
-    SPD_HIP(hipGraphDestroy(g));
-    graph_grid = grid;
-    graph_variant = variant;
+    auto& of_shape = gexec[variant];
+    if (graph_grid[variant] != grid)
+        for (auto& g : of_shape)
+            if (g) { SPD_HIP(hipGraphExecDestroy(g)); g = nullptr; }
+    graph_grid[variant] = grid;
+    hipGraphExec_t& exec = of_shape[plane_shares(variant, grid)];
+    if (!exec)
+    {
+        hipGraph_t g = nullptr;
+        SPD_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+        enqueue_step(ctx->stream);
+        SPD_HIP(hipStreamEndCapture(ctx->stream, &g));
+        SPD_HIP(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
+        SPD_HIP(hipGraphDestroy(g));
+    }
+    return exec;
 }
 
 void Batch::collect_diag(int first_step, int nsteps)
@@ -285,14 +342,15 @@ void Batch::step(int nsteps)
 {
     need(nsteps >= 0, "nsteps must be >= 0");
     if (worklist_dirty) upload_worklist();
+    if (!shape_set) choose_shape();
     int done = 0;
     while (done < nsteps)
     {
         const int chunk = std::min(nsteps - done, hist_len);
-        if (use_graph && (!gexec || graph_grid != grid || graph_variant != variant)) build_graph();
+        const hipGraphExec_t exec = use_graph ? step_graph() : nullptr;
         for (int t = 0; t < chunk; ++t)
         {
-            if (use_graph) SPD_HIP(hipGraphLaunch(gexec, ctx->stream));
+            if (use_graph) SPD_HIP(hipGraphLaunch(exec, ctx->stream));
             else           enqueue_step(ctx->stream);
         }
         collect_diag(host_step, chunk);
@@ -351,6 +409,7 @@ int Batch::tune()
 {
     if (worklist_dirty) upload_worklist();
     if (nwork == 0) return grid;
+    fix_shape();
     // save the step-start state (Q0) of the active slots
     double* save = nullptr;
     SPD_HIP(hipMalloc((void**)&save, sizeof(double)*kSlotDoubles*(size_t)nwork));

@@ -31,8 +31,10 @@ struct Batch
     int hist_len;
     int max_slots = 0, max_cases = 0;
     int num_cu = 1;
-    int grid = 0, graph_grid = -1;
-    int variant = 0, graph_variant = -1;   // stage kernel shape (batch.hpp)
+    int grid = 0;
+    int variant = 0;                 // stage kernel shape (batch.hpp)
+    bool shape_set = false;          // the caller or the tuner chose grid and variant
+    int resident[kBatchShapeVariants] = {};   // workgroups of each shape that run on a CU at once
     bool use_graph = true;
     bool order_interleaved = false;
     bool worklist_dirty = true;
@@ -47,8 +49,10 @@ struct Batch
     int* d_init_slots = nullptr;
     CaseParams* d_cases = nullptr;
     double* d_diag = nullptr;
+    double* d_parts = nullptr;       // unit sums of one step (BatchDev::parts)
     BatchDev dev{};
-    hipGraphExec_t gexec = nullptr;
+    hipGraphExec_t gexec[kBatchShapeVariants][3] = {};   // a step of each shape with 1, 2, 4 plane shares
+    int graph_grid[kBatchShapeVariants] = {};            // and the grid those of a shape were recorded with
     std::vector<int> free_slots, free_tables, h_slot_case, h_nbr, h_worklist, case_of_table;
     std::vector<CaseParams> h_cases;
     std::map<int, BatchCase> cases;
@@ -62,8 +66,11 @@ struct Batch
     int add_case(const spd_case_desc& d);
     void remove_case(int id);
     void upload_worklist();
+    int plane_shares(int v, int g, double* cost = nullptr) const;   // log2 of the shares for the work list
+    void choose_shape();
+    void fix_shape();
     void enqueue_step(hipStream_t s);
-    void build_graph();
+    hipGraphExec_t step_graph();
     void collect_diag(int first_step, int nsteps);
     void step(int nsteps);
     const BatchCase& get(int id) const;

@@ -314,3 +314,33 @@ def test_served_case_that_diverges_is_retired_others_unaffected():
         assert np.array_equal(by[rid].state, st), rid
         assert np.array_equal(by[rid].ke, ke), rid
     assert eng.fits(specs[0]) and eng.fits(specs[1])
+
+
+@pytest.mark.parametrize("grid", [None, 5, 70, 4096])
+def test_plane_shares_agree_bitwise(grid):
+    """The default shape and its 1, 2 or 4 workgroups along a block's planes
+    follow the number of blocks (16 here, then 412); a case's bits do not, nor
+    do its diagnostics, under the graph or launched directly."""
+    spec = sa.CaseSpec("vortex", (32, 64, 32), mach=0.3, reynolds=700.0)
+    b = sa.Batch(512 * MB)
+    b.set_kernel_shape(16, 1, 3)
+    b.set_shape(768)
+    ref = b.add(spec)
+    filler = [b.add(_tgv(48, 3)) for _ in range(28)]
+    b.step(4)
+    assert len(filler) == 28
+    c = sa.Batch(512 * MB)
+    if grid:
+        c.set_shape(grid)
+    cid = c.add(spec)
+    c.step(2)
+    more = [c.add(_tgv(48, 3)) for _ in range(15)]
+    c.step(1)
+    for m in more:
+        c.remove(m)
+    c.use_graph(False)
+    c.step(1)
+    print("plane shares, grid", grid, c.shape(), flush=True)
+    assert np.array_equal(b.download(ref), c.download(cid))
+    for x, y in zip(b.diag(ref), c.diag(cid)):
+        assert len(x) == 4 and np.array_equal(x, y)
