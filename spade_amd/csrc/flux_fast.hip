@@ -717,6 +717,8 @@ bool select_fast(const DevGeom& G, const spd_flux_desc& f, int& keep, int& pd, i
     // identity or diagonal (tanh) maps; a 16 x 16 cross-section
     if (G.nc[0] != 16 || G.nc[1] != 16 || G.ng < 1) return false;
     for (int a = 0; a < 3; ++a) if (G.map_kind[a] != SPD_MAP_IDENTITY && G.map_kind[a] != SPD_MAP_TANH) return false;
+    // the metric tables hold 16 planes; they are not read where only y is mapped
+    if (map_variant(G) == 2 && G.nc[2] > 16) return false;
     if (const char* e = getenv("SPD_DISABLE_FAST")) if (e[0] == '1') return false;
     // terms must be a subsequence of [keep2, pdiss, visc] in that order
     keep = 0; pd = 0; vs = 0;

@@ -120,3 +120,30 @@ def test_weno_quotients_equal_per_cell(p, jump, name):
     print(name, p, jump, np.isnan(out[0]).sum(), flush=True)
     assert np.array_equal(out[0], out[1], equal_nan=True)
     assert np.isfinite(out[0]).all() == np.isfinite(jump)
+
+
+@pytest.mark.parametrize("nz", [16, 17, 40])
+def test_tall_mapped_blocks_equal_per_cell(nz):
+    """16x16 cross-sections with x and z mapped: more than 16 planes exceed the
+    staged kernel's metric tables, so those take the tiled kernel."""
+    import spade_amd as sa
+    g = sa.CartesianGrid((16, 16, nz), (1, 2, 1), ((0.0, 2.0), (-1.0, 1.0), (0.0, 1.5)), num_exch=2,
+                         maps=(sa.tanh_map(0.0, 2.0, 0.8), None, sa.tanh_map(0.0, 1.5, 1.1)))
+    q = np.random.default_rng(nz).standard_normal(g.host_shape)
+    q[..., 0] = (1.0 + 0.02 * q[..., 0]) / GAMMA
+    q[..., 1] = 1.1 * (1.0 + 0.005 * q[..., 1])
+    arr = sa.GridArray(g).upload(q)
+    flux = RawFlux([dict(kind=1, order=2), VC], GAMMA, R)
+    out = []
+    for generic in (False, True):
+        if generic:
+            os.environ["SPD_DISABLE_SPEC"] = os.environ["SPD_DISABLE_FAST"] = "1"
+        try:
+            rhs = sa.GridArray(g)
+            sa.flux_div(arr, rhs, flux)
+            out.append(rhs.download())
+        finally:
+            os.environ.pop("SPD_DISABLE_SPEC", None)
+            os.environ.pop("SPD_DISABLE_FAST", None)
+    print("tall mapped block", nz, flush=True)
+    assert np.array_equal(*out)
