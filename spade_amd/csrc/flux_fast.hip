@@ -112,7 +112,8 @@ struct StageArgs
     double c[3];
     int n;                       // 1..3 coefficients, the last one for L
     int store_rhs;               // also write L to rhs
-    double gamma, R;
+    double gamma, R, inv_gm1;    // inv_gm1 = 1/(gamma - 1)
+    int same_R;                  // R is the flux's gas constant
     const int* push;             // push table (d_push)
     int push_ghosts;             // write the ghosts this stage's result feeds
     const int* nbr;              // source table (d_nbr), read halos from neighbour interiors (STG == 2)
@@ -540,8 +541,15 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
         {
             // the stage of cell (i,j,k): its stored primitives are the window's
             const long long co = own_off + k*plane;
-            double qq[5] = {cur.p, cur.T, cur.u, cur.v, cur.w}, cons[5];
-            p2c(A.gamma, A.R, qq, cons);
+            // p2c and c2p of spd_stage.hpp, their quotients without the ends of
+            // the range; the cell's density is the window's where the stage
+            // converts with the flux's gas constant
+            double rho = cur.rho;
+            if (!A.same_R) rho = quot_inf(cur.p, A.R*cur.T);
+            const double rhoU2 = rho*(cur.u*cur.u + cur.v*cur.v + cur.w*cur.w);
+            const double gm1 = A.gamma - 1.0;
+            double qq[5], cons[5] = {rho, 0.5*rhoU2 + __builtin_amdgcn_div_fixup(div_const(cur.p, gm1, A.inv_gm1), gm1, cur.p),
+                                     rho*cur.u, rho*cur.v, rho*cur.w};
             #pragma unroll
             for (int t = 0; t < 2; ++t)
             {
@@ -561,7 +569,13 @@ k_flux_fast(DevGeom G, const double* __restrict__ prims, double* __restrict__ rh
                 #pragma unroll
                 for (int v = 0; v < 5; ++v) cons[v] += inc[v];
             }
-            c2p(A.gamma, A.R, cons, qq);
+            {
+                const double invrho = quot_inf(1.0, cons[0]);
+                qq[2] = invrho*cons[2]; qq[3] = invrho*cons[3]; qq[4] = invrho*cons[4];
+                const double ru2 = cons[0]*(qq[2]*qq[2] + qq[3]*qq[3] + qq[4]*qq[4]);
+                qq[0] = gm1*(cons[1] - 0.5*ru2);
+                qq[1] = quot_inf(qq[0], A.R*cons[0]);
+            }
             #pragma unroll
             for (int v = 0; v < 5; ++v) __builtin_nontemporal_store(qq[v], A.qout + co + v*sv);
             if (A.push_ghosts)
@@ -823,7 +837,8 @@ bool launch_flux_stage_fast(const Grid& g, const double* qin, double* qout, doub
     for (int t = 0; t < nr; ++t) A.c[t] = coef[t];
     A.n = nr;
     A.store_rhs = store_rhs ? 1 : 0;
-    A.gamma = gamma; A.R = R;
+    A.gamma = gamma; A.R = R; A.inv_gm1 = 1.0/(gamma - 1.0);
+    A.same_R = R == C.R ? 1 : 0;
     A.push = g.d_push;
     A.push_ghosts = push ? 1 : 0;
     A.nbr = g.d_nbr;

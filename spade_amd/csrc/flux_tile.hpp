@@ -78,15 +78,15 @@ __device__ inline TCell derive(const TileCfg& C, const Raw5& r)
     TCell c{r.p, r.T, r.u, r.v, r.w, {0.0, 0.0, 0.0, 0.0}};
     if constexpr (S::extra == 2)
     {
-        c.x[0] = r.p/(C.R*r.T);
-        c.x[1] = r.p/(c.x[0]*C.gm1);
+        c.x[0] = quot_inf(r.p, C.R*r.T);
+        c.x[1] = quot_inf(r.p, c.x[0]*C.gm1);
     }
     else if constexpr (S::conv == CV_WENO || S::conv == CV_FIRST)
     {
         // rusanov_t / phys_flux_t (flux_funcs.h:19-52, 107-124)
         const double k2 = r.u*r.u + r.v*r.v + r.w*r.w;
-        const double rho = r.p/(C.R*r.T);
-        const double pdiff = r.p/rho, ei = r.p/(rho*C.gm1);
+        const double rho = quot_inf(r.p, C.R*r.T);
+        const double pdiff = quot_inf(r.p, rho), ei = quot_inf(r.p, rho*C.gm1);
         c.x[0] = 0.5*rho;
         if (S::conv == CV_WENO && C.split_phys) c.x[2] = 0.5*k2 + pdiff + ei;
         else
@@ -101,9 +101,9 @@ __device__ inline TCell derive(const TileCfg& C, const Raw5& r)
         // fweno_t (convective.h:355-496)
         const double k2 = r.u*r.u + r.v*r.v + r.w*r.w;
         const double RT = C.R*r.T;
-        c.x[0] = r.p/RT;
+        c.x[0] = quot_inf(r.p, RT);
         c.x[3] = (sqrt(k2) + sqrt(RT*C.gamma))*c.x[0]*0.5;
-        c.x[1] = k2*0.5 + RT/C.gm1;
+        c.x[1] = k2*0.5 + quot_inf(RT, C.gm1);
         c.x[2] = c.x[1] + RT;
     }
     return c;
@@ -126,23 +126,6 @@ __device__ inline double split_diss(const TCell& q, int n)
 {
     return n == 0 ? q.x[3] : q.x[3]*(n == 1 ? q.x[1] : (n == 2 ? q.u : (n == 3 ? q.v : q.w)));
 }
-
-// a/b, rounded as the IEEE quotient, where b and the quotient are well inside
-// the normal range: the reciprocal instruction (relative error e <= 2^-22)
-// times 1 + e + e^2 is good to e^3, and one residual step rounds the quotient.
-// 7 instructions; the compiler's division adds two scalings and two fix-ups
-// for the ends of the range, which this needs only through quot_inf.
-__device__ inline double quot(double a, double b)
-{
-    double y = __builtin_amdgcn_rcp(b);
-    const double e = __builtin_fma(-b, y, 1.0);
-    y = __builtin_fma(y, __builtin_fma(e, e, e), y);
-    const double q = a*y;
-    return __builtin_fma(__builtin_fma(-q, b, a), y, q);
-}
-
-// the same with the division's results for zeros, infinities and NaN
-__device__ inline double quot_inf(double a, double b) { return __builtin_amdgcn_div_fixup(quot(a, b), b, a); }
 
 // The candidate values of weno_t and fweno_t.  A product with 1/2 is exact, so
 // fusing it into its sum leaves the one rounding of the per-cell expressions.

@@ -147,3 +147,40 @@ def test_tall_mapped_blocks_equal_per_cell(nz):
             os.environ.pop("SPD_DISABLE_FAST", None)
     print("tall mapped block", nz, flush=True)
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("name", ["keep2", "weno_visc"])
+@pytest.mark.parametrize("cells", [(16, 16, 16), (11, 9, 6)], ids=["staged", "tiled"])
+def test_cell_quotients_equal_per_cell(cells, name):
+    """Densities and energies of cells at the ends: zero, NaN and negative
+    temperatures and pressures (densities zero, infinite, NaN), and far from
+    one.  (Infinite pressures and temperatures themselves the per-cell kernel
+    multiplies by the zero components of a face normal, which the face-once
+    kernels leave out.)"""
+    import spade_amd as sa
+    g = sa.CartesianGrid(cells, (1, 2, 1), ((0.0, 2.0), (-1.0, 1.0), (0.0, 1.5)), num_exch=2)
+    rng = np.random.default_rng(9)
+    q = rng.standard_normal(g.host_shape)
+    q[..., 0] = 1.0 + 0.02 * q[..., 0]
+    q[..., 1] = 1.1 * (1.0 + 0.005 * q[..., 1])
+    pts = [(0.0, 1.0), (1.0, 0.0), (0.0, 0.0), (np.nan, 1.0), (1.0, -2.0), (-1.0, 1.0),
+           (1e200, 1.0), (1e-200, 1.0), (1.0, 1e100), (1.0, 1e-100), (-0.0, 1.0)]
+    for p, t in pts:
+        at = (rng.integers(q.shape[0]),) + tuple(rng.integers(2, n - 2) for n in q.shape[1:4])
+        q[at][:2] = p, t
+    arr = sa.GridArray(g).upload(q)
+    flux = RawFlux([dict(kind=1, order=2), VC] if name == "keep2" else FLUXES[name], GAMMA, R)
+    out = []
+    for generic in (False, True):
+        if generic:
+            os.environ["SPD_DISABLE_SPEC"] = os.environ["SPD_DISABLE_FAST"] = "1"
+        try:
+            rhs = sa.GridArray(g)
+            sa.flux_div(arr, rhs, flux)
+            out.append(rhs.download())
+        finally:
+            os.environ.pop("SPD_DISABLE_SPEC", None)
+            os.environ.pop("SPD_DISABLE_FAST", None)
+    print("cell quotients", name, cells, np.isnan(out[0]).sum(), flush=True)
+    assert np.isnan(out[0]).any() and np.isfinite(out[0]).any()
+    assert np.array_equal(*out, equal_nan=True)
