@@ -888,7 +888,7 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
 // a thread per halo column it loads again and the two closing-face passes (a
 // third of a wave's faces each) -- and workgroups along k by rounds
 // of resident workgroups (as fast_zsplit), a share costing its planes plus
-// about two for its prologue: twelve 4 x 8 x 4 blocks run as 24 workgroups, 27
+// kTilePrologue for its prologue: twelve 4 x 8 x 4 blocks run as 24 workgroups, 27
 // blocks of 32^3 as 432, 240 blocks of 24 x 20 x 12 as 480 of half a block each.
 constexpr double kTilePrologue = 0.65;
 struct TilePlan { int wi, wj, tx, ty, zs, nt; size_t lds; };
