@@ -413,7 +413,8 @@ int spd_flux_div_kernel(spd_array_t prims, const spd_flux_desc* flux, int* kind)
     {
         require(prims && kind, "null argument");
         validate_flux(flux, prims->a.grid->geom.ng);
-        *kind = flux_div_fast_eligible(*prims->a.grid, *flux) ? 1 : (flux_div_spec_code(*flux) ? 2 : 0);
+        const Grid& g = *prims->a.grid;
+        *kind = flux_div_fast_eligible(g, *flux) ? 1 : (flux_div_spec_code(*flux) && tile_offsets_fit(g.geom) ? 2 : 0);
     });
 }
 

@@ -149,6 +149,7 @@ SPD_TILE_DECL(tile_central) SPD_TILE_DECL(tile_pdiss) SPD_TILE_DECL(tile_split) 
 bool launch_flux_div_tile(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
                           hipStream_t s)
 {
+    if (!flux_div_spec_code(f) || !tile_offsets_fit(g.geom)) return false;
     int conv = CV_NONE, pdiss = 0;
     for (int m = 0; m < f.nterms; ++m)
         switch (f.terms[m].kind)
@@ -174,7 +175,7 @@ void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, co
 {
     // compositions with compile-time code run tiled; any other one through the
     // run-time term dispatch, one thread per cell
-    if (flux_div_spec_code(f) && launch_flux_div_tile(g, prims, rhs, f, increment, s)) return;
+    if (launch_flux_div_tile(g, prims, rhs, f, increment, s)) return;
     const DevGeom& G = g.geom;
     const long long nwg = (long long)((G.nc[0] + 15)/16)*((G.nc[1] + 15)/16)*G.nc[2]*G.nblk;
     hipLaunchKernelGGL(k_flux_div_generic, dim3((unsigned)nwg), dim3(256), 0, s, G, prims, rhs, f, pow_of(f),

@@ -112,8 +112,9 @@ __device__ inline void lds_barrier()
 // ---- kernels' host launchers ----
 void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
                              bool increment, hipStream_t s);
-// the tiled kernel for the compositions of flux_div_spec_code on blocks of any
-// size and any coordinates; false (nothing launched) for others
+// the tiled kernel for the compositions of flux_div_spec_code on any
+// coordinates and on blocks of any size whose offsets fit; false (nothing
+// launched) for others
 bool launch_flux_div_tile(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f, bool increment,
                           hipStream_t s);
 bool launch_flux_div_fast(const Grid& g, const double* prims, double* rhs, const spd_flux_desc& f,
@@ -137,8 +138,13 @@ bool launch_flux_stage_fast(const Grid& g, const double* qin, double* qout, doub
                             int wall_mask = 0, double t_wall = 0.0);
 bool flux_stage_fast_eligible(const Grid& g, const spd_flux_desc& f);
 bool stage_reads_neighbours_ok(const Grid& g, int wall_mask);
-// non-zero when the composition has a compile-time specialised per-cell kernel
+// non-zero when the composition has compile-time code (the tiled kernel)
 int flux_div_spec_code(const spd_flux_desc& f);
+// The tiled kernel forms the offsets within a variable of a block in 32 bits (a
+// 64-bit offset per column costs it 2 to 4 registers, and the widest
+// compositions spill them), so a block with more than 2^31 - 1 doubles per
+// variable takes the generic kernel, whose offsets have 64
+inline bool tile_offsets_fit(const DevGeom& G) { return G.sv <= 0x7fffffffLL; }
 // the composition contains a hybrid_scheme_t term
 bool flux_has_hybrid(const spd_flux_desc& f);
 void launch_exchange(const Grid& g, double* a, hipStream_t s);
