@@ -6,6 +6,7 @@
 #pragma once
 #include "spd_internal.hpp"
 #include "pow_series.hpp"
+#include <cmath>
 
 namespace spd {
 namespace {
@@ -41,6 +42,16 @@ inline void cfg_pdiss(FastCfg& C, const spd_flux_term& t, double sc)
     C.eps_p = t.eps_p; C.eps_T = t.eps_T;
 }
 
+// A constant divisor and its reciprocal for div_const, which takes no infinite
+// one (its residual would be 0*inf): 1 with the reciprocal 0 gives the 0 of
+// a/inf (an infinite Prandtl number switches heat conduction off)
+inline void const_divisor(double b, double& d, double& y)
+{
+    const bool inf = std::isinf(b);
+    d = inf ? 1.0 : b;
+    y = inf ? 0.0 : 1.0/b;
+}
+
 inline void cfg_visc(FastCfg& C, const spd_flux_term& t, double sc)
 {
     // constant law (viscous_laws.h:77-99): beta = -2 mu / 3, alpha = mu / Pr
@@ -48,8 +59,9 @@ inline void cfg_visc(FastCfg& C, const spd_flux_term& t, double sc)
     C.visc2_s = sc*double(-2.0*t.mu/3.0);
     C.cond_s = C.spec_heat*(sc*(t.mu*(1.0/t.prandtl)));
     // power law (viscous_laws.h:121-134)
-    C.mu_ref_s = sc*t.mu; C.T_ref = t.T_ref; C.power = t.power; C.prandtl = t.prandtl;
-    C.inv_T_ref = 1.0/t.T_ref; C.inv_prandtl = 1.0/t.prandtl;
+    C.mu_ref_s = sc*t.mu; C.power = t.power;
+    const_divisor(t.T_ref, C.T_ref, C.inv_T_ref);
+    const_divisor(t.prandtl, C.prandtl, C.inv_prandtl);
     C.t_ref_one = (t.T_ref == 1.0);
     C.ps = PowSeries::make(t.power);
 }
