@@ -890,42 +890,64 @@ k_flux_div_spec_tile(DevGeom G, const double* __restrict__ prims, double* __rest
 // of resident workgroups (as fast_zsplit), a share costing its planes plus
 // kTilePrologue for its prologue: twelve 4 x 8 x 4 blocks run as 24 workgroups, 27
 // blocks of 32^3 as 432, 240 blocks of 24 x 20 x 12 as 480 of half a block each.
+//
+// The search runs on every call, so it steps from one tile side (and one share
+// of planes) to the next smaller one and not through every count of tiles,
+// most of which leave the side as it is: some hundred candidates for any
+// block.  One by one, a 512 x 512 x 2 block cost 226 us of host time a call, more than
+// three times what its {KEEP2} residual takes, and a 2048 x 2048 x 2 one 3500 us.
 constexpr double kTilePrologue = 0.65;
 struct TilePlan { int wi, wj, tx, ty, zs, nt; size_t lds; };
 
+inline int ceil_div(int a, int b) { return (a + b - 1)/b; }
+
+// the least number of parts of n that makes the largest smaller than part (n + 1: none does)
+inline int parts_below(int n, int part) { return part > 1 ? ceil_div(n, part - 1) : n + 1; }
+
+// threads of a tile's workgroup
+inline int tile_threads(int H, int wi, int wj) { return 64*ceil_div(std::max(wi*wj, 2*H*(wi + wj) + 4), 64); }
+
+// cost of the tiles of a cross-section in threads, infinite where a tile has too many
+inline double tile_cost(const DevGeom& G, int H, int wi, int wj)
+{
+    const int nt = tile_threads(H, wi, wj);
+    if (nt > 256) return 1e300;
+    return (double)ceil_div(G.nc[0], wi)*ceil_div(G.nc[1], wj)*(nt + 0.25*(2*H*(wi + wj) + 4) + 128.0/3.0);
+}
+
+// cost of a tiling's planes shared out to zs workgroups
+inline double share_cost(const DevGeom& G, const TilePlan& p, int zs, size_t lds, int cus)
+{
+    const int per_cu = std::max(1, std::min((int)(160*1024/(lds + 2048)), 512/p.nt));
+    const double rounds = std::ceil((double)p.tx*p.ty*G.nblk*zs/((double)per_cu*cus));
+    return rounds*(ceil_div(G.nc[2], zs) + kTilePrologue);
+}
+
 inline TilePlan plan_tile(const DevGeom& G, int H, int SS, bool map, int cus)
 {
-    auto ceil_div = [](int a, int b) { return (a + b - 1)/b; };
     TilePlan best{};
-    double best_cost = 1e300;
-    for (int tx = ceil_div(G.nc[0], 64); tx <= ceil_div(G.nc[0], 4); ++tx)
+    double best_cost = 1e299;
+    const int nx = G.nc[0], ny = G.nc[1], nz = G.nc[2];
+    for (int tx = ceil_div(nx, 64), wi; tx <= ceil_div(nx, 4); tx = parts_below(nx, wi))
     {
-        const int wi = ceil_div(G.nc[0], tx);
-        for (int ty = ceil_div(G.nc[1], std::min(64, std::max(1, 256/wi))); ty <= ceil_div(G.nc[1], 1); ++ty)
+        wi = ceil_div(nx, tx);
+        for (int ty = ceil_div(ny, std::min(64, 256/wi)), wj; ty <= ny; ty = parts_below(ny, wj))
         {
-            const int wj = ceil_div(G.nc[1], ty);
-            if (wi*wj > 256) continue;
-            const int halo = 2*H*(wi + wj) + 4;
-            const int nt = 64*ceil_div(std::max(wi*wj, halo), 64);
-            if (nt > 256) continue;
-            const double cost = (double)ceil_div(G.nc[0], wi)*ceil_div(G.nc[1], wj)*(nt + 0.25*halo + 128.0/3.0);
+            wj = ceil_div(ny, ty);
+            const double cost = tile_cost(G, H, wi, wj);
             if (cost < best_cost - 1e-9)
             {
                 best_cost = cost;
-                best = TilePlan{wi, wj, ceil_div(G.nc[0], wi), ceil_div(G.nc[1], wj), 1, nt, 0};
+                best = TilePlan{wi, wj, ceil_div(nx, wi), ceil_div(ny, wj), 1, tile_threads(H, wi, wj), 0};
             }
         }
     }
-    const int nz = G.nc[2];
-    const double tiles = (double)best.tx*best.ty*G.nblk;
     best_cost = 1e300;
-    for (int zs = ceil_div(nz, 64); zs <= nz; ++zs)
+    for (int zs = ceil_div(nz, 64), share; zs <= nz; zs = parts_below(nz, share))
     {
-        const int share = ceil_div(nz, zs);
+        share = ceil_div(nz, zs);
         const size_t lds = sizeof(double)*(size_t)TileLds(best.wi, best.wj, share, H, SS, map).total;
-        const int per_cu = std::max(1, std::min((int)(160*1024/(lds + 2048)), 512/best.nt));
-        const double rounds = std::ceil(tiles*zs/((double)per_cu*cus));
-        const double cost = rounds*(share + kTilePrologue);
+        const double cost = share_cost(G, best, zs, lds, cus);
         if (cost < best_cost - 1e-9) { best_cost = cost; best.zs = zs; best.lds = lds; }
     }
     return best;
