@@ -88,7 +88,9 @@ void validate_flux(const spd_flux_desc* f, int ng)
 
 // Host arrays in the reference layout (AoS, variable fastest) cross the
 // boundary through a device staging buffer of a few blocks; the layout is
-// converted by a kernel, so the host only copies contiguous bytes.
+// converted by a kernel, so the host only copies contiguous bytes.  The buffer
+// belongs to the grid, whose arrays several host threads may copy: copy_mu is held
+// from here until the buffer's last use is queued.
 double* ensure_stage(Grid& g)
 {
     if (!g.d_stage)
@@ -892,6 +894,7 @@ void upload_blocks(spd_array_s* arr, int lb0, int nb, const double* host, bool s
 {
     Grid& g = *arr->a.grid;
     require(lb0 >= 0 && nb >= 0 && lb0 + nb <= g.geom.nblk, "block range outside the grid");
+    std::unique_lock<std::mutex> lock(g.ctx->copy_mu);
     double* stage = ensure_stage(g);
     const long long cells = (long long)g.geom.N[0]*g.geom.N[1]*g.geom.N[2];
     for (int b0 = lb0; b0 < lb0 + nb; b0 += g.stage_blocks)
@@ -901,6 +904,7 @@ void upload_blocks(spd_array_s* arr, int lb0, int nb, const double* host, bool s
                                g.ctx->stream));
         launch_aos_to_soa(g, stage, arr->a.d, b0, n, g.ctx->stream);
     }
+    lock.unlock();                // (what is queued on the stream stays in order)
     if (sync) SPD_HIP(hipStreamSynchronize(g.ctx->stream));
 }
 
@@ -908,12 +912,11 @@ void download_blocks(const spd_array_s* arr, int lb0, int nb, double* host, bool
 {
     Grid& g = *arr->a.grid;
     require(lb0 >= 0 && nb >= 0 && lb0 + nb <= g.geom.nblk, "block range outside the grid");
+    std::unique_lock<std::mutex> lock(g.ctx->copy_mu);
     double* stage = ensure_stage(g);
     const long long cells = (long long)g.geom.N[0]*g.geom.N[1]*g.geom.N[2];
     // (a caller that does not wait brings pinned memory of its own)
     const bool large = sync && sizeof(double)*5*cells*nb >= kDownLarge;
-    std::unique_lock<std::mutex> lock(g.ctx->copy_mu, std::defer_lock);
-    if (large) lock.lock();
     for (int b0 = lb0; b0 < lb0 + nb; b0 += g.stage_blocks)
     {
         const int n = std::min(g.stage_blocks, lb0 + nb - b0);
@@ -923,6 +926,7 @@ void download_blocks(const spd_array_s* arr, int lb0, int nb, double* host, bool
         if (large) copy_down(*g.ctx, (char*)h, (const char*)stage, bytes, g.ctx->stream);
         else SPD_HIP(hipMemcpyAsync(h, stage, bytes, hipMemcpyDeviceToHost, g.ctx->stream));
     }
+    lock.unlock();
     if (sync) SPD_HIP(hipStreamSynchronize(g.ctx->stream));
 }
 

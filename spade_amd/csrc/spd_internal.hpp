@@ -58,8 +58,9 @@ struct Ctx
     size_t h_io_doubles = 0;
     hipEvent_t io_ev[2] = {nullptr, nullptr};
     // pinned slots of large downloads, one per copying thread (api.cpp),
-    // allocated on first use and freed with the context; the mutex is held for
-    // a whole download
+    // allocated on first use and freed with the context.  The mutex guards them
+    // and the staging buffers of the context's grids: it is held while an upload
+    // or download queues its work, which for a large download is until its end
     static constexpr int kCopyThreads = 4;
     static constexpr size_t kCopySlot = 4u << 20;
     std::mutex copy_mu;

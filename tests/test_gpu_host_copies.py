@@ -43,3 +43,34 @@ def test_two_threads_one_context():
     for t in threads:
         t.join()
     assert ok == [True, True]
+
+
+@pytest.mark.parametrize("other", ["up", "up_and_down"])
+def test_threads_on_arrays_of_one_grid(other):
+    """The arrays of a grid share its staging buffer: one host thread downloads
+    a large array over and over while another uploads (and downloads) its own."""
+    import spade_amd as sa
+    g = sa.CartesianGrid((16, 16, 16), (4, 4, 4), ((0.0, 1.0),) * 3)
+    rng = np.random.default_rng(7)
+    host = [rng.standard_normal(g.host_shape) for _ in range(2)]
+    arr = [sa.GridArray(g).upload(h) for h in host]
+    ok = [True, True]
+
+    def down():
+        for _ in range(12):
+            ok[0] = ok[0] and np.array_equal(arr[0].download(), host[0])
+
+    def up_and_down():
+        for n in range(12):
+            h = host[1] * (1.0 + n)
+            arr[1].upload(h)
+            if other == "up_and_down":
+                ok[1] = ok[1] and np.array_equal(arr[1].download(), h)
+    threads = [threading.Thread(target=down), threading.Thread(target=up_and_down)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    print(other, ok, flush=True)
+    assert ok == [True, True]
+    assert np.array_equal(arr[1].download(), host[1] * 12.0)
