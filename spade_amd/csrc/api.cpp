@@ -7,8 +7,6 @@
 #include <algorithm>
 #include <atomic>
 #include <memory>
-#include <system_error>
-#include <thread>
 #include <utility>
 
 namespace spd {
@@ -846,44 +844,32 @@ double map_coord(const spd_map1d& m, double xi)
     return c + h*std::tanh(m.beta*((xi - c)/h))/std::tanh(m.beta);
 }
 
-// A large copy from the device staging buffer to pageable host memory, by
-// kCopyThreads threads of this call, each moving every kCopyThreads-th piece
-// through its own pinned slot: the DMA engine runs at its pinned rate (55 GB/s)
-// while the other threads copy from the slots to the caller's memory, which
-// one pageable hipMemcpyAsync does in turn (17 GB/s).  Two pieces a thread
-// where that makes them 1 to 4 MiB: every piece costs some 30 us of calls (20.5
-// MB in 512 KiB pieces 1030 us, in 2 MiB ones 650).  Complete on return.  (Up,
-// the pageable copy stays: it reaches 35 GB/s on warm pages, and pieces were
-// 5 ms slower on 100 MB of pages just written.)
-static void copy_down(Ctx& c, char* host, const char* dev, size_t bytes, hipStream_t s)
+// The device side of copy_in_pieces: pieces of a device buffer through the
+// context's pinned slots, queued on its stream.  (Up, the pageable copy stays: it
+// reaches 35 GB/s on warm pages, and pieces were 5 ms slower on 100 MB of pages just
+// written.)
+struct DownCopy
 {
-    constexpr int T = Ctx::kCopyThreads;
-    const size_t piece = std::min(Ctx::kCopySlot, std::max<size_t>(1u << 20, ((bytes/(2*T) + 65535) >> 16) << 16));
-    if (!c.copy_slot) SPD_HIP(hipHostMalloc((void**)&c.copy_slot, T*Ctx::kCopySlot));
-    for (auto& e : c.copy_ev) if (!e) SPD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    std::atomic<int> failed{(int)hipSuccess};
-    auto work = [&](int t)
+    Ctx& c;
+    const char* dev;
+    std::atomic<int> error{(int)hipSuccess};
+
+    bool ok(hipError_t e) { if (e != hipSuccess) error = (int)e; return e == hipSuccess; }
+    const char* slot(int t) const { return c.copy_slot + t*CopyShape::slot; }
+    bool fetch(int t, size_t off, size_t n)
     {
-        auto ok = [&](hipError_t e) { if (e != hipSuccess) failed = (int)e; return e == hipSuccess; };
-        if (!ok(hipSetDevice(c.device))) return;
-        char* slot = c.copy_slot + t*Ctx::kCopySlot;
-        for (size_t off = t*piece; off < bytes && failed == (int)hipSuccess; off += T*piece)
-        {
-            const size_t n = std::min(piece, bytes - off);
-            if (!ok(hipMemcpyAsync(slot, dev + off, n, hipMemcpyDeviceToHost, s))) return;
-            if (!ok(hipEventRecord(c.copy_ev[t], s)) || !ok(hipEventSynchronize(c.copy_ev[t]))) return;
-            std::memcpy(host + off, slot, n);
-        }
-    };
-    std::thread helper[T - 1];
-    for (int t = 1; t < T; ++t)
-    {
-        try { helper[t - 1] = std::thread(work, t); }
-        catch (const std::system_error&) { work(t); }    // no thread to be had: the pieces in turn
+        return ok(hipSetDevice(c.device))
+            && ok(hipMemcpyAsync(c.copy_slot + t*CopyShape::slot, dev + off, n, hipMemcpyDeviceToHost, c.stream))
+            && ok(hipEventRecord(c.copy_ev[t], c.stream)) && ok(hipEventSynchronize(c.copy_ev[t]));
     }
-    work(0);
-    for (auto& h : helper) if (h.joinable()) h.join();
-    if (failed != (int)hipSuccess) throw HipError{(hipError_t)(int)failed, "host array copy"};
+};
+
+static void copy_down(Ctx& c, char* host, const char* dev, size_t bytes)
+{
+    if (!c.copy_slot) SPD_HIP(hipHostMalloc((void**)&c.copy_slot, CopyShape::threads*CopyShape::slot));
+    for (auto& e : c.copy_ev) if (!e) SPD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    DownCopy d{c, dev};
+    if (!copy_in_pieces(d, host, bytes)) throw HipError{(hipError_t)(int)d.error, "host array copy"};
 }
 
 // Size from which a host array goes that way: 20.5 MB takes 1171 us as one
@@ -923,7 +909,7 @@ void download_blocks(const spd_array_s* arr, int lb0, int nb, double* host, bool
         launch_soa_to_aos(g, arr->a.d, stage, b0, n, g.ctx->stream);
         const size_t bytes = sizeof(double)*5*cells*n;
         double* h = host + 5*cells*(b0 - lb0);
-        if (large) copy_down(*g.ctx, (char*)h, (const char*)stage, bytes, g.ctx->stream);
+        if (large) copy_down(*g.ctx, (char*)h, (const char*)stage, bytes);
         else SPD_HIP(hipMemcpyAsync(h, stage, bytes, hipMemcpyDeviceToHost, g.ctx->stream));
     }
     lock.unlock();

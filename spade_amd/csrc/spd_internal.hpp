@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <mutex>
 #include "../../include/spade_amd.h"
+#include "host_copy.hpp"
 
 namespace spd {
 
@@ -57,15 +58,13 @@ struct Ctx
     double* h_io[2] = {nullptr, nullptr};
     size_t h_io_doubles = 0;
     hipEvent_t io_ev[2] = {nullptr, nullptr};
-    // pinned slots of large downloads, one per copying thread (api.cpp),
+    // pinned slots of large downloads, one per copying thread,
     // allocated on first use and freed with the context.  The mutex guards them
     // and the staging buffers of the context's grids: it is held while an upload
     // or download queues its work, which for a large download is until its end
-    static constexpr int kCopyThreads = 4;
-    static constexpr size_t kCopySlot = 4u << 20;
     std::mutex copy_mu;
-    char* copy_slot = nullptr;            // kCopyThreads slots of kCopySlot bytes
-    hipEvent_t copy_ev[kCopyThreads] = {};
+    char* copy_slot = nullptr;            // CopyShape::threads slots of CopyShape::slot bytes
+    hipEvent_t copy_ev[CopyShape::threads] = {};
 };
 
 struct Grid

@@ -1,0 +1,63 @@
+// Host check of the large downloads' control flow (host_copy.hpp) on a device
+// that is a host buffer.  argv: scenario, bytes; prints "result bytes_equal pieces".
+#include <cstdio>
+#include <cstdlib>
+#include <mutex>
+#include <new>
+#include <string>
+#include <system_error>
+#include <vector>
+#include "../../spade_amd/csrc/host_copy.hpp"
+
+static int threads_left = 1 << 30;
+static bool refuse_with_bad_alloc = false;
+
+// std::thread that is refused after threads_left of them
+struct FewThreads
+{
+    std::thread t;
+    FewThreads() = default;
+    template <class F> explicit FewThreads(F f)
+    {
+        if (threads_left-- <= 0)
+        {
+            if (refuse_with_bad_alloc) throw std::bad_alloc();
+            throw std::system_error(std::make_error_code(std::errc::resource_unavailable_try_again));
+        }
+        t = std::thread(f);
+    }
+    bool joinable() const { return t.joinable(); }
+    void join() { t.join(); }
+};
+
+struct Fake
+{
+    std::vector<char> dev;
+    std::vector<std::vector<char>> slots{(size_t)spd::CopyShape::threads};
+    std::atomic<int> pieces{0};
+    long fail_at = -1;
+    const char* slot(int t) const { return slots[t].data(); }
+    bool fetch(int t, size_t off, size_t n)
+    {
+        if (n > spd::CopyShape::slot || pieces++ == fail_at) return false;
+        slots[t].assign(dev.begin() + off, dev.begin() + off + n);
+        return true;
+    }
+};
+
+int main(int, char** argv)
+{
+    const std::string scenario = argv[1];
+    const size_t bytes = std::strtoull(argv[2], nullptr, 10);
+    Fake f;
+    f.dev.resize(bytes);
+    for (size_t n = 0; n < bytes; ++n) f.dev[n] = (char)(n*2654435761u >> 13);
+    if (scenario == "no_thread") threads_left = 0;
+    if (scenario == "one_thread") threads_left = 1;
+    if (scenario == "no_memory") { threads_left = 1; refuse_with_bad_alloc = true; }
+    if (scenario == "failing_piece") f.fail_at = 2;
+    std::vector<char> host(bytes);
+    const bool r = spd::copy_in_pieces<FewThreads>(f, host.data(), bytes);
+    std::printf("%d %d %d\n", (int)r, (int)(host == f.dev), (int)f.pieces);
+    return 0;
+}

@@ -1,0 +1,37 @@
+"""Large downloads where something is refused (CPU only): the control flow of
+spade_amd/csrc/host_copy.hpp with a host buffer for the device."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path_factory.mktemp("copy") / "copy_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", os.path.join(HERE, "native", "copy_check.cpp"), "-o", exe],
+                   check=True)
+
+    def go(scenario, nbytes):
+        r = subprocess.run([exe, scenario, str(nbytes)], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, (r.returncode, r.stderr[-300:])
+        return [int(x) for x in r.stdout.split()]
+    return go
+
+
+@pytest.mark.parametrize("nbytes", [1, (4 << 20) + 3, (20 << 20) + 5, 67 << 20])
+@pytest.mark.parametrize("scenario", ["all", "no_thread", "one_thread", "no_memory"])
+def test_threads_refused(run, scenario, nbytes):
+    """Whatever refuses a thread, every piece arrives and the running threads end."""
+    result, equal, pieces = run(scenario, nbytes)
+    assert result and equal and pieces >= 1
+
+
+def test_failing_piece_is_reported(run):
+    result, _, pieces = run("failing_piece", 67 << 20)
+    assert not result and pieces < 17
