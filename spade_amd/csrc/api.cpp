@@ -855,6 +855,15 @@ struct DownCopy
     std::atomic<int> error{(int)hipSuccess};
 
     bool ok(hipError_t e) { if (e != hipSuccess) error = (int)e; return e == hipSuccess; }
+    bool slots()
+    {
+        bool have = c.copy_slot || hipHostMalloc((void**)&c.copy_slot, CopyShape::threads*CopyShape::slot) == hipSuccess;
+        if (!have) c.copy_slot = nullptr;
+        for (auto& e : c.copy_ev)
+            if (have && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; have = false; }
+        if (!have) (void)hipGetLastError();      // not an error of this call
+        return have;
+    }
     const char* slot(int t) const { return c.copy_slot + t*CopyShape::slot; }
     bool fetch(int t, size_t off, size_t n)
     {
@@ -864,12 +873,13 @@ struct DownCopy
     }
 };
 
-static void copy_down(Ctx& c, char* host, const char* dev, size_t bytes)
+// false, nothing copied: no pinned memory to be had
+static bool copy_down(Ctx& c, char* host, const char* dev, size_t bytes)
 {
-    if (!c.copy_slot) SPD_HIP(hipHostMalloc((void**)&c.copy_slot, CopyShape::threads*CopyShape::slot));
-    for (auto& e : c.copy_ev) if (!e) SPD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     DownCopy d{c, dev};
-    if (!copy_in_pieces(d, host, bytes)) throw HipError{(hipError_t)(int)d.error, "host array copy"};
+    const Copied r = copy_in_pieces(d, host, bytes);
+    if (r == Copied::failed) throw HipError{(hipError_t)(int)d.error, "host array copy"};
+    return r == Copied::all;
 }
 
 // Size from which a host array goes that way: 20.5 MB takes 1171 us as one
@@ -909,8 +919,8 @@ void download_blocks(const spd_array_s* arr, int lb0, int nb, double* host, bool
         launch_soa_to_aos(g, arr->a.d, stage, b0, n, g.ctx->stream);
         const size_t bytes = sizeof(double)*5*cells*n;
         double* h = host + 5*cells*(b0 - lb0);
-        if (large) copy_down(*g.ctx, (char*)h, (const char*)stage, bytes);
-        else SPD_HIP(hipMemcpyAsync(h, stage, bytes, hipMemcpyDeviceToHost, g.ctx->stream));
+        if (large && copy_down(*g.ctx, (char*)h, (const char*)stage, bytes)) continue;
+        SPD_HIP(hipMemcpyAsync(h, stage, bytes, hipMemcpyDeviceToHost, g.ctx->stream));
     }
     lock.unlock();
     if (sync) SPD_HIP(hipStreamSynchronize(g.ctx->stream));

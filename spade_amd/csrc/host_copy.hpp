@@ -17,6 +17,8 @@ struct CopyShape
     static constexpr size_t slot = 4u << 20;
 };
 
+enum class Copied { all, failed, no_slots };
+
 // Copies `bytes` to host: thread t of CopyShape::threads (0 is the caller's)
 // moves every threads-th piece, Api::fetch(t, off, n) bringing the n bytes from
 // offset off into slot(t).  The DMA engine runs at its pinned rate (55 GB/s)
@@ -24,11 +26,13 @@ struct CopyShape
 // one pageable hipMemcpyAsync does in turn (17 GB/s).  Two pieces a thread where that
 // makes them 1 to 4 MiB: every piece costs some 30 us of calls (20.5 MB in
 // 512 KiB pieces 1030 us, in 2 MiB ones 650).  The pieces of a thread that cannot
-// be had are copied here, in turn.  False when a fetch failed (Api keeps the reason);
-// complete otherwise.
+// be had are copied here, in turn.
+// failed: a fetch did (Api keeps the reason).  no_slots: Api::slots() has none to
+// offer, nothing was copied and the caller takes another way.
 template <class Thread = std::thread, class Api>
-bool copy_in_pieces(Api& api, char* host, size_t bytes)
+Copied copy_in_pieces(Api& api, char* host, size_t bytes)
 {
+    if (!api.slots()) return Copied::no_slots;
     constexpr int T = CopyShape::threads;
     const size_t piece = std::min(CopyShape::slot, std::max<size_t>(1u << 20, ((bytes/(2*T) + 65535) >> 16) << 16));
     std::atomic<bool> failed{false};
@@ -50,7 +54,7 @@ bool copy_in_pieces(Api& api, char* host, size_t bytes)
     }
     work(0);
     for (auto& h : helper) if (h.joinable()) h.join();
-    return !failed;
+    return failed ? Copied::failed : Copied::all;
 }
 
 } // namespace spd

@@ -33,14 +33,16 @@ struct FewThreads
 struct Fake
 {
     std::vector<char> dev;
-    std::vector<std::vector<char>> slots{(size_t)spd::CopyShape::threads};
+    std::vector<std::vector<char>> mem{(size_t)spd::CopyShape::threads};
     std::atomic<int> pieces{0};
     long fail_at = -1;
-    const char* slot(int t) const { return slots[t].data(); }
+    bool have_slots = true;
+    bool slots() const { return have_slots; }
+    const char* slot(int t) const { return mem[t].data(); }
     bool fetch(int t, size_t off, size_t n)
     {
         if (n > spd::CopyShape::slot || pieces++ == fail_at) return false;
-        slots[t].assign(dev.begin() + off, dev.begin() + off + n);
+        mem[t].assign(dev.begin() + off, dev.begin() + off + n);
         return true;
     }
 };
@@ -56,8 +58,10 @@ int main(int, char** argv)
     if (scenario == "one_thread") threads_left = 1;
     if (scenario == "no_memory") { threads_left = 1; refuse_with_bad_alloc = true; }
     if (scenario == "failing_piece") f.fail_at = 2;
+    if (scenario == "no_slots") f.have_slots = false;
     std::vector<char> host(bytes);
-    const bool r = spd::copy_in_pieces<FewThreads>(f, host.data(), bytes);
-    std::printf("%d %d %d\n", (int)r, (int)(host == f.dev), (int)f.pieces);
+    const spd::Copied r = spd::copy_in_pieces<FewThreads>(f, host.data(), bytes);
+    const char* name = r == spd::Copied::all ? "all" : r == spd::Copied::failed ? "failed" : "no_slots";
+    std::printf("%s %d %d\n", name, (int)(host == f.dev), (int)f.pieces);
     return 0;
 }

@@ -20,7 +20,8 @@ def run(tmp_path_factory):
     def go(scenario, nbytes):
         r = subprocess.run([exe, scenario, str(nbytes)], capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, (r.returncode, r.stderr[-300:])
-        return [int(x) for x in r.stdout.split()]
+        result, equal, pieces = r.stdout.split()
+        return result, int(equal), int(pieces)
     return go
 
 
@@ -29,9 +30,16 @@ def run(tmp_path_factory):
 def test_threads_refused(run, scenario, nbytes):
     """Whatever refuses a thread, every piece arrives and the running threads end."""
     result, equal, pieces = run(scenario, nbytes)
-    assert result and equal and pieces >= 1
+    assert result == "all" and equal and pieces >= 1
 
 
 def test_failing_piece_is_reported(run):
     result, _, pieces = run("failing_piece", 67 << 20)
-    assert not result and pieces < 17
+    assert result == "failed" and pieces < 17
+
+
+def test_no_pinned_memory(run):
+    """Refused pinned memory copies nothing and says so: the caller goes on with
+    the pageable copy."""
+    result, equal, pieces = run("no_slots", 20 << 20)
+    assert (result, equal, pieces) == ("no_slots", 0, 0)
