@@ -855,20 +855,25 @@ struct DownCopy
     std::atomic<int> error{(int)hipSuccess};
 
     bool ok(hipError_t e) { if (e != hipSuccess) error = (int)e; return e == hipSuccess; }
+    // (the events belong to the context's device; the caller's own one stays)
     bool slots()
     {
+        int callers = c.device;
+        (void)hipGetDevice(&callers);
+        if (callers != c.device) (void)hipSetDevice(c.device);
         bool have = c.copy_slot || hipHostMalloc((void**)&c.copy_slot, CopyShape::threads*CopyShape::slot) == hipSuccess;
         if (!have) c.copy_slot = nullptr;
         for (auto& e : c.copy_ev)
             if (have && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; have = false; }
+        if (callers != c.device) (void)hipSetDevice(callers);
         if (!have) (void)hipGetLastError();      // not an error of this call
         return have;
     }
     const char* slot(int t) const { return c.copy_slot + t*CopyShape::slot; }
+    bool enter() { return ok(hipSetDevice(c.device)); }
     bool fetch(int t, size_t off, size_t n)
     {
-        return ok(hipSetDevice(c.device))
-            && ok(hipMemcpyAsync(c.copy_slot + t*CopyShape::slot, dev + off, n, hipMemcpyDeviceToHost, c.stream))
+        return ok(hipMemcpyAsync(c.copy_slot + t*CopyShape::slot, dev + off, n, hipMemcpyDeviceToHost, c.stream))
             && ok(hipEventRecord(c.copy_ev[t], c.stream)) && ok(hipEventSynchronize(c.copy_ev[t]));
     }
 };

@@ -28,7 +28,8 @@ enum class Copied { all, failed, no_slots };
 // 512 KiB pieces 1030 us, in 2 MiB ones 650).  The pieces of a thread that cannot
 // be had are copied here, in turn.
 // failed: a fetch did (Api keeps the reason).  no_slots: Api::slots() has none to
-// offer, nothing was copied and the caller takes another way.
+// offer, nothing was copied and the caller takes another way.  Api::enter() sets up
+// a helper thread (its device) and is not called in the caller's.
 template <class Thread = std::thread, class Api>
 Copied copy_in_pieces(Api& api, char* host, size_t bytes)
 {
@@ -36,8 +37,10 @@ Copied copy_in_pieces(Api& api, char* host, size_t bytes)
     constexpr int T = CopyShape::threads;
     const size_t piece = std::min(CopyShape::slot, std::max<size_t>(1u << 20, ((bytes/(2*T) + 65535) >> 16) << 16));
     std::atomic<bool> failed{false};
+    const std::thread::id caller = std::this_thread::get_id();
     auto work = [&](int t) noexcept
     {
+        if (std::this_thread::get_id() != caller && !api.enter()) { failed = true; return; }
         for (size_t off = t*piece; off < bytes && !failed; off += T*piece)
         {
             const size_t n = std::min(piece, bytes - off);

@@ -1,5 +1,7 @@
 // Host check of the large downloads' control flow (host_copy.hpp) on a device
-// that is a host buffer.  argv: scenario, bytes; prints "result bytes_equal pieces".
+// that is a host buffer.  argv: scenario, bytes; prints
+// "result bytes_equal pieces entered callers", the threads that entered the device
+// and whether the caller's is one of them.
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
@@ -38,6 +40,9 @@ struct Fake
     long fail_at = -1;
     bool have_slots = true;
     bool slots() const { return have_slots; }
+    std::mutex mu;
+    std::vector<std::thread::id> entered;
+    bool enter() { std::lock_guard<std::mutex> l(mu); entered.push_back(std::this_thread::get_id()); return true; }
     const char* slot(int t) const { return mem[t].data(); }
     bool fetch(int t, size_t off, size_t n)
     {
@@ -62,6 +67,7 @@ int main(int, char** argv)
     std::vector<char> host(bytes);
     const spd::Copied r = spd::copy_in_pieces<FewThreads>(f, host.data(), bytes);
     const char* name = r == spd::Copied::all ? "all" : r == spd::Copied::failed ? "failed" : "no_slots";
-    std::printf("%s %d %d\n", name, (int)(host == f.dev), (int)f.pieces);
+    const bool callers = std::count(f.entered.begin(), f.entered.end(), std::this_thread::get_id()) > 0;
+    std::printf("%s %d %d %zu %d\n", name, (int)(host == f.dev), (int)f.pieces, f.entered.size(), (int)callers);
     return 0;
 }
