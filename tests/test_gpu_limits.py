@@ -17,7 +17,8 @@ WALE = dict(sgs=1, sgs_cw=0.5, sgs_delta=0.3, sgs_prt=0.9)
 def _both(cells, terms, ng=2, maps=(None, None, None), touch=None):
     """The residual from the kernel the library chooses and from the generic one."""
     import spade_amd as sa
-    g = sa.CartesianGrid(cells, (2, 1, 1), ((0.0, 2.0), (-1.0, 1.0), (0.0, 1.5)), num_exch=ng, maps=maps)
+    g = sa.CartesianGrid(cells, (2, 1, 1), ((0.0, 2.0), (-1.0, 1.0), (0.0, 1.5)), num_exch=ng,
+                         maps=tuple(None if m is None else sa.tanh_map(*m) for m in maps))
     q = np.random.default_rng(sum(cells)).standard_normal(g.host_shape)
     q[..., 0] = (1.0 + 0.02 * q[..., 0]) / GAMMA
     q[..., 1] = 1.1 * (1.0 + 0.005 * q[..., 1])
@@ -53,3 +54,19 @@ def test_infinite_parameters(changes, cells):
     got, ref = _both(cells, [dict(kind=1, order=2), dict(POWER, **changes)])
     assert np.all(np.isfinite(ref))
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("cells", [(16, 16, 16), (11, 9, 6)], ids=["staged", "tiled"])
+@pytest.mark.parametrize("var", [2, 3, 4])
+def test_infinite_velocity_on_a_stretched_axis(var, cells):
+    """An infinite velocity gradient divided by dy/deta stays infinite, so the
+    Ducros sensor's denominator gives the finite values that the division gives:
+    wherever the generic kernel's residual is a number, so is this one, and the
+    same one."""
+    def touch(q):
+        q[1, 5, 6, 7, var] = np.inf
+    pdiss = dict(kind=3, sensor=1, sensor_param=1e-6, eps_p=0.1, eps_T=0.05)
+    got, ref = _both(cells, [dict(kind=1, order=2), pdiss], maps=(None, (-1.0, 1.0, 1.5), None), touch=touch)
+    assert np.isnan(ref).any()
+    number = ~np.isnan(ref)
+    assert np.array_equal(got[number], ref[number])
