@@ -116,7 +116,7 @@ void advance_generic(spd_integrator_s* it)
     if (it->trans == SPD_TRANS_PRIM_CONS)
     {
         // transform-aware advance (advance.h:233-280)
-        const bool push = !it->bcfn;
+        const bool push = !it->bcfn && stage_pushes(g.geom);
         auto advance_to = [&](int prev, int curr)
         {
             const double* rr[SPD_RK_MAX_STAGES];
@@ -126,8 +126,8 @@ void advance_generic(spd_integrator_s* it)
                 rr[j] = it->res[j]->a.d;
                 coef[j] = row_diff(tb, curr, prev, j)*dt;   // zero entries are skipped by the kernel
             }
-            // with the caller's own bc the exchange may not be what follows, so
-            // the ghosts are left to it
+            // (with the caller's own bc the exchange may not be what follows, so
+            // the ghosts are left to it)
             launch_rk_transform_stage(g, q->a.d, rr, coef, S, it->gamma, it->R, st, push);
         };
         eval_stage(it, 0, q, false);

@@ -198,6 +198,21 @@ __host__ __device__ inline long long stored_offset(const DevGeom& g, int i, int 
     return g.xh + (long long)section*g.N[1]*g.N[2] + row;
 }
 
+// Whether the stage launch of a Butcher-table step writes the ghosts it feeds
+// or leaves them to an exchange.  It saves the exchange its launch and its
+// reads of what the stage has just written, and pays with scattered writes,
+// most of them across x.  Measured per stage, pushed and exchanged: 24x20x12
+// blocks (5x6x8) 40 and 56 us, 128^3 45 and 58, 12 blocks of 4x8x4 5.8 and 7.4,
+// 512 of 4^3 7.8 and 10.5; but 27000 blocks of 2^3 185 and 110, 512 of 6x32x32
+// 152 and 145, 256 of 8x8x256 232 and 205, 8000 of 5x6x7 195 and 168.  Hence where rows are
+// long and few cells are ghosts, or all of it stays in the caches; of 197
+// shapes none lost 2 %.
+inline bool stage_pushes(const DevGeom& G)
+{
+    const double cells = (double)G.nc[0]*G.nc[1]*G.nc[2], ratio = (double)G.sv/cells;
+    return (G.nc[0] >= 12 && ratio < 2.8) || (G.nc[0] >= 4 && ratio <= 8.0 && (double)G.sv*G.nblk < 1.5e6);
+}
+
 // d x / d xi of a diagonal map along axis d at computational coordinate xi
 // (core/coord_system.h:103-140): 1 for identity axes, for the tanh
 // stretching x = c + h tanh(beta s)/tanh(beta), s = (xi - c)/h:

@@ -1,10 +1,11 @@
-// Host check of the tiled flux_div's launch.  Commands on the input, one per
+// Host check of the tiled flux_div's launch and of rules on block shapes.  Commands on the input, one per
 // line, with a block of nx ny nz cells and ng ghost layers each:
 //   offsets nx ny nz ng          whether the kernel's 32-bit offsets fit the block, and
 //                                whether every stored cell's offset within a variable does
 //   plan nx ny nz ng blocks H SS map   the plan: wi wj tx ty zs threads bytes of LDS, and whether an
 //                                exhaustive search of the same costs finds the same one
 //   time nx ny nz ng             microseconds of one plan
+//   pushes nx ny nz ng blocks    whether a Butcher-table stage writes the ghosts it feeds
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -83,6 +84,12 @@ int main()
             const bool same = p.wi == q.wi && p.wj == q.wj && p.tx == q.tx && p.ty == q.ty && p.zs == q.zs
                 && p.nt == q.nt && p.lds == q.lds;
             std::printf("%d %d %d %d %d %d %zu %d\n", p.wi, p.wj, p.tx, p.ty, p.zs, p.nt, p.lds, (int)same);
+        }
+        else if (!std::strcmp(cmd, "pushes"))
+        {
+            int nblk;
+            if (std::scanf("%d", &nblk) != 1) return 1;
+            std::printf("%d\n", (int)stage_pushes(block(nc, ng, nblk)));
         }
         else
         {

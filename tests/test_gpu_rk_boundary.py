@@ -41,8 +41,8 @@ def _advance(sa, cells, blocks, walls, table, callback):
 
 @pytest.mark.parametrize("walls", sorted(WALLS))
 @pytest.mark.parametrize("cells, blocks", [((16, 16, 8), (2, 2, 1)), ((16, 16, 16), (1, 1, 2)), ((3, 5, 4), (2, 1, 3)),
-                                           ((2, 2, 2), (1, 2, 2)), ((11, 9, 6), (2, 2, 2))],
-                         ids=["16x16x8", "16x16x16", "3x5x4", "2x2x2", "11x9x6"])
+                                           ((2, 2, 2), (1, 2, 2)), ((11, 9, 6), (2, 2, 2)), ((16, 3, 3), (1, 2, 2))],
+                         ids=["16x16x8", "16x16x16", "3x5x4", "2x2x2", "11x9x6", "16x3x3"])
 def test_default_boundary_equals_callback(cells, blocks, walls):
     import spade_amd as sa
     for table in ("rk4", "ssprk3_table"):

@@ -1,4 +1,4 @@
-"""Host side of the tiled flux_div (CPU only): tests/native/tile_check.cpp
+"""Host side of the tiled flux_div and rules on block shapes (CPU only): tests/native/tile_check.cpp
 compiled for the host with hipcc."""
 import os
 import random
@@ -71,3 +71,13 @@ def test_plan_costs_no_time(check, cells):
     (us, ok), = check("time", [cells + (2,)])
     print(cells, us)
     assert ok and us < 50.0
+
+
+def test_stage_pushes_where_measured_faster(check):
+    """The ghosts of a Butcher-table stage: pushed and exchanged times in us."""
+    rows = [((24, 20, 12, 2, 240), 40, 56), ((128, 128, 128, 2, 1), 45, 58), ((4, 8, 4, 2, 12), 5.8, 7.4),
+            ((4, 4, 4, 2, 512), 7.8, 10.5), ((16, 16, 16, 2, 512), 71, 90), ((40, 48, 64, 2, 2), 8.7, 12.8),
+            ((2, 2, 2, 2, 27000), 185, 110), ((6, 32, 32, 2, 512), 152, 145), ((8, 8, 256, 2, 256), 232, 205),
+            ((5, 6, 7, 2, 8000), 195, 168), ((2, 8, 8, 2, 216), 11.3, 9.7), ((14, 8, 8, 2, 3375), 231, 198)]
+    got = [bool(p) for p, in check("pushes", [r[0] for r in rows])]
+    assert got == [pushed < exchanged for _, pushed, exchanged in rows]
