@@ -191,7 +191,7 @@ def rows_measure(sa, g, q, exch, gas, flux, reps=10):
 def compositions_measure(sa, blocks=8, reps=10):
     """flux_div of the compositions outside the LDS-staged kernel's set on the
     TGV (blocks^3 blocks of 16^3 cells, identity coordinates): the
-    compile-time specialised per-cell kernel against the generic one with
+    tiled kernel with compile-time code against the generic per-cell one with
     run-time term dispatch (SPD_DISABLE_SPEC=1), mean of reps launches after
     three untimed ones.  The two give the same bits."""
     nb, nc, ng = (blocks,) * 3, (16, 16, 16), 2
@@ -358,7 +358,7 @@ def main():
     ap.add_argument("--channel", action="store_true",
                     help="instead of the benchmark: time flux_div on the 192x128x96 stretched channel only")
     ap.add_argument("--compositions", action="store_true",
-                    help="instead of the benchmark: other flux compositions on the 128^3 TGV, specialised "
+                    help="instead of the benchmark: other flux compositions on the 128^3 TGV, tiled kernel "
                          "vs generic per-cell kernel")
     args = ap.parse_args()
     if args.channel:

@@ -1,8 +1,10 @@
 // LDS-staged flux_div for the hot combinations on gfx950:
 //   cent_keep<2> [+ pressure_diss_lr (const | Ducros)] [+ visc_lr (const | power law)]
-// on identity coordinates and blocks with a 16x16 (i,j) cross-section.
+// on identity or diagonal (tanh) coordinates and blocks with a 16x16 (i,j)
+// cross-section.
 //
-// One workgroup (256 threads, thread (i,j)) owns one block and marches over k.
+// One workgroup (256 threads, thread (i,j)) owns a block, or a share of its
+// planes, and marches over k.
 // Every face flux is evaluated once: thread (i,j) evaluates the low x-face
 // i-1/2, the low y-face j-1/2 and the high z-face k+1/2 of its cell; the 16
 // block-boundary x-faces and the 16 y-faces of a plane are evaluated by 16
@@ -725,7 +727,7 @@ bool dispatch_visc_stage(int visc, const Grid& g, const double* qin, double* rhs
 
 namespace {
 
-// Selects the fast kernel for (grid, flux); false when the generic kernel must run.
+// Selects the fast kernel for (grid, flux); false when the tiled or the generic kernel runs.
 bool select_fast(const DevGeom& G, const spd_flux_desc& f, int& keep, int& pd, int& vs, FastCfg& C)
 {
     // identity or diagonal (tanh) maps; a 16 x 16 cross-section
@@ -753,7 +755,7 @@ bool select_fast(const DevGeom& G, const spd_flux_desc& f, int& keep, int& pd, i
         }
         else if (t.kind == SPD_TERM_VISC && stage < 3)
         {
-            if (t.sgs != SPD_SGS_NONE) return false;   // the per-cell kernels evaluate subgrid models
+            if (t.sgs != SPD_SGS_NONE) return false;   // the tiled kernel evaluates subgrid models
             vs = 1 + t.law; stage = 3;
             cfg_visc(C, t, sc);
             if (t.law == SPD_LAW_POWER && !(t.T_ref > 0.0 && t.prandtl > 0.0)) return false;

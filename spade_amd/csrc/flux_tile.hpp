@@ -14,21 +14,25 @@
 // gathering its stencil (and, mapped, its tanh metrics) again from memory
 // through a run-time index, at one wave per SIMD.  Measured per flux_div,
 // before and now: cent_keep<2> + visc_lr on 5 x 6 x 8 blocks of 24 x 20 x 12,
-// 2549 -> 73 us; WENO + visc_lr on 128^3, 2594 -> 246 us; cent_keep<4> + WALE on
-// 96^3 in 32^3 blocks, 602 -> 95 us; WENO + visc_lr on 80 x 48 x 64 stretched
-// cells, 798 -> 55 us; twelve blocks of 4 x 8 x 4, 72.7 -> 11.4 us.
+// 2549 -> 67 us; WENO + visc_lr on 128^3, 2594 -> 211 us; cent_keep<4> + WALE on
+// 96^3 in 32^3 blocks, 602 -> 88 us; WENO + visc_lr on 80 x 48 x 64 stretched
+// cells, 798 -> 43 us; twelve blocks of 4 x 8 x 4, 72.7 -> 6.8 us.
 //
 // LDS holds the velocities of planes k-1, k, k+1 (ring of three) and, of plane
 // k, p, T and the per-cell quantities the composition's faces share (rho, e;
 // the split coefficients of WENO): what a face needs of a neighbour is computed
 // once per cell.  Records are interleaved per cell with an odd stride (3, and
 // 3, 5 or 7 doubles), so a row of lanes reads LDS without bank conflicts and
-// the offsets of a cell's x-neighbours and components are immediates.  The
-// window of the widest composition is 73 KB: two workgroups per CU.
+// the offsets of a cell's x-neighbours and components are immediates.  With a
+// 16 x 16 tile the window of the widest composition takes 73 KB, two workgroups per
+// CU; longer and narrower tiles up to 90 KB, one.
 //
 // Arithmetic: the expressions of flux_cell.hpp in the same order, with the
 // components of a diagonal map's face normal that are zero left out, so for
-// finite states the result equals the per-cell code's bit for bit.
+// finite states the result equals the per-cell code's bit for bit.  (The per-cell
+// code multiplies those components by the velocities and the pressure, so around an
+// infinite one it gives NaN at faces where this gives an infinity or, in the
+// outputs that do not contain it, a number.)
 #pragma once
 #include "spd_internal.hpp"
 #include "flux_face.hpp"
@@ -143,9 +147,11 @@ __device__ inline double weno_lin(double u0, double u1, double u2, double d1, do
 }
 
 // weno_t's smooth weights (convective.h:275-332).  The b are at least 1e-16,
-// so the squares lie in [1e-32, inf] and the a in [0, 1e32]: a division by a
-// square needs the infinite case only, the weights' own divisions neither end
-// (both a 0, where both squares overflow, is NaN either way).  Six divisions
+// so the squares start at 1e-32 and the a end at 1e32: a division by a square
+// needs the infinite case only, the weights' own divisions neither end.  That
+// holds for squares up to 1e290 (split fluxes 1e72 apart) and for infinite ones
+// (both a 0 is NaN either way); in the decade before overflow, where an a is
+// subnormal, a weight may differ from the division's.  Six divisions
 // a component were 40 % of the kernel's instructions: a 128^3 grid of
 // {WENO, viscous} 247 -> 218 us with these, same bits.
 __device__ inline double weno_smooth(double u0, double u1, double u2, double d1, double d2, double d3)
