@@ -74,3 +74,39 @@ def test_threads_on_arrays_of_one_grid(other):
     print(other, ok, flush=True)
     assert ok == [True, True]
     assert np.array_equal(arr[1].download(), host[1] * 12.0)
+
+
+def test_pinned_destination():
+    """A download into memory that is pinned already goes there directly: the
+    same values (also at an odd place in the buffer), in less time than pageable
+    memory takes, whose pieces pass through pinned slots (0.64 of it at 20 MB)."""
+    import ctypes as C
+    import time
+    import spade_amd as sa
+    lib = sa.load()
+    g = sa.CartesianGrid((16, 16, 16), (4, 4, 4), ((0.0, 1.0),) * 3)
+    host = np.random.default_rng(5).standard_normal(g.host_shape)
+    a = sa.GridArray(g).upload(host)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    hip.hipHostFree.argtypes = [C.c_void_p]
+    mem = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(mem), host.nbytes + 24, 0) == 0
+    try:
+        pinned = np.ctypeslib.as_array(C.cast(mem, C.POINTER(C.c_double)), shape=(host.size + 3,))
+        pinned[:] = 0.0
+        plain = np.zeros(host.size)
+        best = {}
+        for name, out in (("pinned", pinned[3:]), ("pageable", plain)):
+            times = []
+            for _ in range(20):
+                t0 = time.perf_counter()
+                assert lib.spd_array_download(a._h, out.ctypes.data_as(C.POINTER(C.c_double))) == 0
+                times.append(time.perf_counter() - t0)
+            best[name] = min(times)
+            assert np.array_equal(out, host.ravel())
+        print(best, flush=True)
+        assert np.all(pinned[:3] == 0.0)
+        assert best["pinned"] < 0.85 * best["pageable"]
+    finally:
+        hip.hipHostFree(mem)
